@@ -47,18 +47,18 @@ __device__ int EU_RANGE_FAULT;
 #define EU_EXACT 0
 #endif
 
-__device__ __forceinline__ bool eu_pos_in_range(double v) { return v >= 0x1p-120 && v <= 0x1p120; }
+/* (`&` and `|`: short-circuit evaluation compiled to a chain of branches) */
+__device__ __forceinline__ bool eu_pos_in_range(double v) { return (v >= 0x1p-120) & (v <= 0x1p120); }
 
 __device__ __forceinline__ bool eu_mom_in_range(double v)
 {
     const double a = fabs(v);
-    return a <= 0x1p120 && (a >= 0x1p-400 || a == 0.0);
+    return (a <= 0x1p120) & ((a >= 0x1p-400) | (a == 0.0));
 }
 
 __device__ __forceinline__ bool eu_in_range(double r, double m, double n, double e, double p)
 {
-    return eu_pos_in_range(r) && eu_pos_in_range(e) && eu_pos_in_range(p) && eu_mom_in_range(m) &&
-           eu_mom_in_range(n);
+    return eu_pos_in_range(r) & eu_pos_in_range(e) & eu_pos_in_range(p) & eu_mom_in_range(m) & eu_mom_in_range(n);
 }
 
 /* flag a state outside the range (a vector store; a benign race: every
@@ -95,14 +95,17 @@ __device__ __forceinline__ eu_q eu_at(const S &s, int i)
 
 /*
  * Division.  n/d is formed as the gfx950 compiler's IEEE double division
- * forms it -- reciprocal estimate, two Newton-Raphson refinements, product,
- * one residual correction, special-case fix-up -- less its operand-scaling
- * steps, which leave every value unchanged unless an operand lies within
- * 2^53 of the subnormal range, d is subnormal or the exponents differ by 768
- * or more (no Euler state comes near).  The quotient is therefore bitwise
- * the one `n / d` gives.  The refined reciprocal depends on d alone, so the
- * quotients of one face that share a denominator share it (6 reciprocals
- * serve the 19 quotients of a face).
+ * forms it -- reciprocal estimate, refinement, product, one residual
+ * correction, special-case fix-up -- less its operand-scaling steps, which
+ * leave every value unchanged unless an operand lies within 2^53 of the
+ * subnormal range, d is subnormal or the exponents differ by 768 or more (no
+ * Euler state comes near).  The estimate's relative error e (about 2^-23 at
+ * most) is removed to third order, y + y*(e + e*e), in three instructions
+ * (two Newton steps take four): the reciprocal is 1/d to within 2^-68 before
+ * its final rounding, and the residual correction makes the quotient the
+ * correctly rounded one, bitwise the one `n / d` gives.  The refined
+ * reciprocal depends on d alone, so the quotients that share a denominator
+ * share it.
  */
 struct eu_rcp {
     double d, y; /* denominator, refined reciprocal */
@@ -110,14 +113,27 @@ struct eu_rcp {
 
 __device__ __forceinline__ eu_rcp eu_recip(double d)
 {
-    double y = __builtin_amdgcn_rcp(d);
-    double e = __builtin_fma(-d, y, 1.0);
-    y = __builtin_fma(y, e, y);
-    e = __builtin_fma(-d, y, 1.0);
-    y = __builtin_fma(y, e, y);
+    const double y = __builtin_amdgcn_rcp(d);
+    const double e = __builtin_fma(-d, y, 1.0);
     eu_rcp q;
     q.d = d;
-    q.y = y;
+    q.y = __builtin_fma(y, __builtin_fma(e, e, e), y);
+    return q;
+}
+
+/* The reciprocal of d from an estimate y of it, good to 2^-45.  One Newton
+ * step leaves 1/d less up to 2^-90; the 2^-88 added to the residual puts the
+ * value above 1/d instead.  That matters for a significand of all ones,
+ * d = 2^k (1 - 2^-53), as the densities of a uniform stream are: its
+ * reciprocal lies 2^-106 above the midpoint of two numbers, and rounded
+ * down it would make 2^j/d one ulp too small (the reciprocal instruction
+ * returns the upper number there for the same reason).  Of every other d
+ * either neighbour gives the correctly rounded quotients. */
+__device__ __forceinline__ eu_rcp eu_recip_from(double d, double y)
+{
+    eu_rcp q;
+    q.d = d;
+    q.y = __builtin_fma(y, __builtin_fma(-d, y, 1.0) + 0x1p-88, y);
     return q;
 }
 
@@ -172,60 +188,137 @@ __device__ __forceinline__ double eu_sqrt(double x)
     return (x == 0.0 || x == __builtin_inf()) ? x : g;
 }
 
-/* gM1*(E - (m*m + n*n)/(2*rho))  (euler.py:284-293); r2 is the reciprocal
- * of 2*rho */
-__device__ __forceinline__ double eu_pressure(const eu_q &q, const eu_rcp &r2)
+/* sqrt(x) and the reciprocals of x and (to about 2^-44) of sqrt(x), for a
+ * density x in the range above.  The square root is eu_sqrt's without its
+ * special cases; its refinement also gives 1/sqrt(x), whose square is the
+ * estimate of 1/x, so a density costs one transcendental instruction (a
+ * quarter of the issue rate) instead of two. */
+struct eu_root {
+    double s, y; /* sqrt(x), estimate of 1/sqrt(x) */
+    eu_rcp rx;   /* reciprocal of x */
+};
+
+__device__ __forceinline__ eu_root eu_sqrt_recip(double x)
 {
-    return GAM_M1 * (q.e - eu_quo_pos(q.m * q.m + q.n * q.n, r2));
+    eu_root o;
+    if (EU_EXACT) {
+        o.s = sqrt(x);
+        o.y = 1.0 / o.s;
+        o.rx = eu_recip(x);
+        return o;
+    }
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = y * 0.5;
+    const double r = __builtin_fma(-h, g, 0.5);
+    h = __builtin_fma(h, r, h);
+    g = __builtin_fma(g, r, g);
+    double d = __builtin_fma(-g, g, x);
+    g = __builtin_fma(d, h, g);
+    d = __builtin_fma(-g, g, x);
+    o.s = __builtin_fma(d, h, g);
+    o.y = h + h;
+    o.rx = eu_recip_from(x, o.y * o.y);
+    return o;
+}
+
+/* gM1*(E - (m*m + n*n)/(2*rho))  (euler.py:284-293); rr is the reciprocal
+ * of rho.  Halving is exact, so the quotient by 2*rho is half the one by rho
+ * and its subtraction one fused operation; likewise below wherever a
+ * product with 0.5 is added (EU_EXACT keeps the written order: its states
+ * may be near the subnormal range, where halving rounds). */
+__device__ __forceinline__ double eu_pressure(const eu_q &q, const eu_rcp &rr)
+{
+    const double k = q.m * q.m + q.n * q.n;
+    if (EU_EXACT)
+        return GAM_M1 * (q.e - eu_quo(k, eu_twice(rr)));
+    return GAM_M1 * __builtin_fma(-0.5, eu_quo_pos(k, rr), q.e);
 }
 
 __device__ __forceinline__ double eu_pressure(const eu_q &q)
 {
-    return eu_pressure(q, eu_recip(2 * q.r));
+    return eu_pressure(q, eu_recip(q.r));
 }
 
-/* q1 + min(Pr,1)/2*(q2-q1), Pr = num/den zeroed when nan, inf, >1e6 or <0
- * (euler.py:250-256) */
-__device__ __forceinline__ eu_q eu_limit(const eu_q &q1, const eu_q &q2, double num, double den)
+/* min(Pr, 1) with Pr = num/den zeroed when nan, inf, >1e6 or <0
+ * (euler.py:250-256).  A zero denominator gives NaN here, which the clamp to
+ * [0, 1] turns into 0 as it does negative ratios. */
+__device__ __forceinline__ double eu_ratio(double num, const eu_rcp &den)
 {
-    double pr = eu_quo(num, eu_recip(den));
-    if (isnan(pr) || isinf(pr) || pr > 1e6 || pr < 0) pr = 0.0;
-    const double h = (1.0 < pr ? 1.0 : pr) / 2;
-    eu_q o;
-    o.r = q1.r + h * (q2.r - q1.r);
-    o.m = q1.m + h * (q2.m - q1.m);
-    o.n = q1.n + h * (q2.n - q1.n);
-    o.e = q1.e + h * (q2.e - q1.e);
+    if (EU_EXACT) {
+        const double pr = eu_quo(num, den);
+        if (isnan(pr) || isinf(pr) || pr > 1e6 || pr < 0) return 0.0;
+        return 1.0 < pr ? 1.0 : pr;
+    }
+    const double pr = eu_quo_pos(num, den);
+    const double c = __builtin_fmin(__builtin_fmax(pr, 0.0), 1.0);
+    /* above 1e6 c is 1.0, whose low word is zero: only the high word changes */
+    const long long b = __double_as_longlong(c);
+    const int hi = pr > 1e6 ? 0 : (int)(b >> 32);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)b);
+}
+
+/* q + c/2*d and q - c/2*d (the limited states of a face's two sides: d is
+ * the difference of its cells, the same for both) */
+__device__ __forceinline__ double eu_add_half(double q, double c, double d)
+{
+    return EU_EXACT ? q + c / 2 * d : __builtin_fma(0.5, c * d, q);
+}
+
+__device__ __forceinline__ double eu_sub_half(double q, double c, double d)
+{
+    return EU_EXACT ? q + c / 2 * -d : __builtin_fma(-0.5, c * d, q);
+}
+
+/* one side's part of a face's central flux, along the first (XDIR) or second
+ * momentum: a = m*m/rho, p the pressure, c = m*n/rho, e = (E+p)*m/rho */
+struct eu_side {
+    double a, p, c, e;
+};
+
+template <bool XDIR>
+__device__ __forceinline__ eu_side eu_flux_side(const eu_q &q, const eu_rcp &rr)
+{
+    eu_side o;
+    const double m = XDIR ? q.m : q.n;
+    o.p = eu_pressure(q, rr);
+    o.a = eu_quo_pos(m * m, rr);
+    o.c = eu_quo_pos(q.m * q.n, rr);
+    o.e = eu_quo_pos((q.e + o.p) * m, rr);
     return o;
 }
 
-/* central flux of a face, x direction (euler.py:181-197) or y (225-241);
- * rl, rr are the reciprocals of L.r and R.r */
+/* Flux f and dissipation d of the face between cells a (low) and b (high),
+ * cl and cr the limiter's ratios of its two sides (eu_ratio):
+ * states q1 + min(Pr,1)/2*(q2-q1) (euler.py:250-256), central flux in x
+ * (euler.py:181-197) or y (225-241), and the spectral radius of the Roe
+ * average, zeroed when nan, times (L - R) (euler.py:258-282).
+ * Bound by FP64 issue: about 200 instructions, four of them transcendental
+ * (three square-root estimates and 1/(sl + sr); the reciprocals of the L, R
+ * and Roe densities come from their roots), for 17 quotients.  Against
+ * reciprocal instructions and two Newton steps for every denominator,
+ * separate limiter differences per side and halvings as operations of their
+ * own, a band-kernel cell and stage went from 605 to 482 VALU instructions:
+ * Euler 1024^2 72.2 -> 57.2 us a step, 2048^2 FP32 state 223 -> 175, standard
+ * kernel 1000 x 1500 108 -> 92.6, bitwise equal. */
 template <bool XDIR>
-__device__ __forceinline__ eu_q eu_flux(const eu_q &L, const eu_q &R, const eu_rcp &rl, const eu_rcp &rr)
+__device__ __forceinline__ void eu_face_vals(const eu_q &a, const eu_q &b, double cl, double cr, eu_q &f, eu_q &d)
 {
-    const double pl = eu_pressure(L, eu_twice(rl)), pr = eu_pressure(R, eu_twice(rr));
-    eu_q f;
-    if (XDIR) {
-        f.r = L.m + R.m;
-        f.m = eu_quo_pos(L.m * L.m, rl) + pl + eu_quo_pos(R.m * R.m, rr) + pr;
-        f.n = eu_quo_pos(L.m * L.n, rl) + eu_quo_pos(R.m * R.n, rr);
-        f.e = eu_quo_pos((L.e + pl) * L.m, rl) + eu_quo_pos((R.e + pr) * R.m, rr);
-    } else {
-        f.r = L.n + R.n;
-        f.m = eu_quo_pos(L.m * L.n, rl) + eu_quo_pos(R.m * R.n, rr);
-        f.n = eu_quo_pos(L.n * L.n, rl) + pl + eu_quo_pos(R.n * R.n, rr) + pr;
-        f.e = eu_quo_pos((L.e + pl) * L.n, rl) + eu_quo_pos((R.e + pr) * R.n, rr);
+    eu_q L, R;
+    {
+        const double dr = b.r - a.r, dm = b.m - a.m, dn = b.n - a.n, de = b.e - a.e;
+        L.r = eu_add_half(a.r, cl, dr); R.r = eu_sub_half(b.r, cr, dr);
+        L.m = eu_add_half(a.m, cl, dm); R.m = eu_sub_half(b.m, cr, dm);
+        L.n = eu_add_half(a.n, cl, dn); R.n = eu_sub_half(b.n, cr, dn);
+        L.e = eu_add_half(a.e, cl, de); R.e = eu_sub_half(b.e, cr, de);
     }
-    return f;
-}
-
-/* spectral radius of the Roe average times (L - R); radius zeroed when nan
- * (euler.py:258-282) */
-template <bool XDIR>
-__device__ __forceinline__ eu_q eu_dissipation(const eu_q &L, const eu_q &R, const eu_rcp &rl, const eu_rcp &rr)
-{
-    const double sl = eu_sqrt(L.r), sr = eu_sqrt(R.r);
+    const eu_root wl = eu_sqrt_recip(L.r), wr = eu_sqrt_recip(R.r);
+    const eu_rcp &rl = wl.rx, &rr = wr.rx;
+    const eu_side l = eu_flux_side<XDIR>(L, rl), r = eu_flux_side<XDIR>(R, rr);
+    f.r = XDIR ? L.m + R.m : L.n + R.n;
+    (XDIR ? f.m : f.n) = l.a + l.p + r.a + r.p;
+    (XDIR ? f.n : f.m) = l.c + r.c;
+    f.e = l.e + r.e;
+    const double sl = wl.s, sr = wr.s;
     const double den = eu_quo_pos(1.0, eu_recip(sl + sr));
     const double a0 = sl * sr;
     const double a1 = (sl * eu_quo_pos(L.m, rl) + sr * eu_quo_pos(R.m, rr)) * den;
@@ -236,19 +329,59 @@ __device__ __forceinline__ eu_q eu_dissipation(const eu_q &L, const eu_q &R, con
     roe.m = a0 * a1;
     roe.n = a0 * a2;
     roe.e = a0 * a3;
-    const eu_rcp ra = eu_recip(a0);
-    double rad = eu_sqrt(eu_quo_pos(GAMMA * eu_pressure(roe, eu_twice(ra)), ra)) + fabs(XDIR ? a1 : a2);
-    if (isnan(rad)) rad = 0.0;
-    eu_q d;
+    const eu_rcp ra = eu_recip_from(a0, wl.y * wr.y);
+    /* a negative Roe pressure gives NaN, of which fmax takes the 0 */
+    const double rad =
+        __builtin_fmax(eu_sqrt(eu_quo_pos(GAMMA * eu_pressure(roe, ra), ra)) + fabs(XDIR ? a1 : a2), 0.0);
     d.r = rad * (L.r - R.r);
     d.m = rad * (L.m - R.m);
     d.n = rad * (L.n - R.n);
     d.e = rad * (L.e - R.e);
-    return d;
+}
+
+/* b + h*(ax*0.5*dt/dx + ay*0.5*dt/dy), the update of one variable from its
+ * two flux sums; h is 1 (final stage) or 0.5 */
+template <bool FINAL>
+__device__ __forceinline__ double eu_update(double b, double ax, double ay)
+{
+    if (EU_EXACT) {
+        const double s = ax * 0.5 * DTDX + ay * 0.5 * DTDY;
+        return FINAL ? b + s : b + 0.5 * s;
+    }
+    const double s = ax * (0.5 * DTDX) + ay * (0.5 * DTDY);
+    return FINAL ? b + s : __builtin_fma(0.5, s, b);
+}
+
+template <bool FINAL>
+__device__ __forceinline__ eu_q eu_update(const eu_q &b, const eu_q &ax, const eu_q &ay)
+{
+    eu_q o;
+    o.r = eu_update<FINAL>(b.r, ax.r, ay.r);
+    o.m = eu_update<FINAL>(b.m, ax.m, ay.m);
+    o.n = eu_update<FINAL>(b.n, ax.n, ay.n);
+    o.e = eu_update<FINAL>(b.e, ax.e, ay.e);
+    return o;
+}
+
+/* flux + dissipation of the face on a cell's low side, less those of the
+ * face on its high side in turn: (fa + da) - fb - db */
+__device__ __forceinline__ eu_q eu_sum(const eu_q &f, const eu_q &d)
+{
+    eu_q o;
+    o.r = f.r + d.r; o.m = f.m + d.m; o.n = f.n + d.n; o.e = f.e + d.e;
+    return o;
+}
+
+__device__ __forceinline__ eu_q eu_less(const eu_q &a, const eu_q &f, const eu_q &d)
+{
+    eu_q o;
+    o.r = a.r - f.r - d.r; o.m = a.m - f.m - d.m; o.n = a.n - f.n - d.n; o.e = a.e - f.e - d.e;
+    return o;
 }
 
 /* flux difference along one direction (euler.py:158-179, 202-223): the
- * west face's flux and dissipation added, the east face's subtracted, *0.5 */
+ * west face's flux and dissipation added, the east face's subtracted (the
+ * factor 0.5 is in eu_update) */
 template <bool XDIR, class S>
 __device__ __forceinline__ eu_q eu_divergence(const S *s, int idx, int stride)
 {
@@ -261,28 +394,13 @@ __device__ __forceinline__ eu_q eu_divergence(const S *s, int idx, int stride)
     eu_range_check(c.r, c.m, c.n, c.e, pc);
     eu_range_check(e.r, e.m, e.n, e.e, pe);
     eu_range_check(ee.r, ee.m, ee.n, ee.e, pee);
-    eu_q acc;
-    acc.r = acc.m = acc.n = acc.e = 0.0;
-
-    eu_q L = eu_limit(w, c, pc - pw, pw - pww);
-    eu_q R = eu_limit(c, w, pc - pw, pe - pc);
-    eu_rcp rl = eu_recip(L.r), rr = eu_recip(R.r);
-    eu_q f = eu_flux<XDIR>(L, R, rl, rr);
-    acc.r = acc.r + f.r; acc.m = acc.m + f.m; acc.n = acc.n + f.n; acc.e = acc.e + f.e;
-    f = eu_dissipation<XDIR>(L, R, rl, rr);
-    acc.r = acc.r + f.r; acc.m = acc.m + f.m; acc.n = acc.n + f.n; acc.e = acc.e + f.e;
-
-    L = eu_limit(c, e, pe - pc, pc - pw);
-    R = eu_limit(e, c, pe - pc, pee - pe);
-    rl = eu_recip(L.r);
-    rr = eu_recip(R.r);
-    f = eu_flux<XDIR>(L, R, rl, rr);
-    acc.r = acc.r - f.r; acc.m = acc.m - f.m; acc.n = acc.n - f.n; acc.e = acc.e - f.e;
-    f = eu_dissipation<XDIR>(L, R, rl, rr);
-    acc.r = acc.r - f.r; acc.m = acc.m - f.m; acc.n = acc.n - f.n; acc.e = acc.e - f.e;
-
-    acc.r = acc.r * 0.5; acc.m = acc.m * 0.5; acc.n = acc.n * 0.5; acc.e = acc.e * 0.5;
-    return acc;
+    const double dw = pc - pw, de = pe - pc;
+    const eu_rcp yw = eu_recip(dw), ye = eu_recip(de);
+    eu_q f, d;
+    eu_face_vals<XDIR>(w, c, eu_ratio(dw, eu_recip(pw - pww)), eu_ratio(dw, ye), f, d);
+    const eu_q acc = eu_sum(f, d);
+    eu_face_vals<XDIR>(c, e, eu_ratio(de, yw), eu_ratio(de, eu_recip(pee - pe)), f, d);
+    return eu_less(acc, f, d);
 }
 
 /* midpoint RK2 (euler.py:131-151): final stages (even globalTimeStep) start
@@ -295,19 +413,13 @@ __device__ __forceinline__ void eu_step(R *shared_state, int idx, int globalTime
     const eu_q fx = eu_divergence<true>(shared_state, idx, SY);
     const eu_q fy = eu_divergence<false>(shared_state, idx, 1);
     R *out = shared_state + idx + TIMES;
-    const eu_q b = eu_at(shared_state, globalTimeStep % 2 == 0 ? idx - TIMES : idx);
-    const double h = globalTimeStep % 2 == 0 ? 1.0 : 0.5;
-    if (globalTimeStep % 2 == 0) {
-        out[0] = (R)(b.r + (fx.r * DTDX + fy.r * DTDY));
-        out[VARS] = (R)(b.m + (fx.m * DTDX + fy.m * DTDY));
-        out[2 * VARS] = (R)(b.n + (fx.n * DTDX + fy.n * DTDY));
-        out[3 * VARS] = (R)(b.e + (fx.e * DTDX + fy.e * DTDY));
-    } else {
-        out[0] = (R)(b.r + h * (fx.r * DTDX + fy.r * DTDY));
-        out[VARS] = (R)(b.m + h * (fx.m * DTDX + fy.m * DTDY));
-        out[2 * VARS] = (R)(b.n + h * (fx.n * DTDX + fy.n * DTDY));
-        out[3 * VARS] = (R)(b.e + h * (fx.e * DTDX + fy.e * DTDY));
-    }
+    const bool fin = globalTimeStep % 2 == 0;
+    const eu_q b = eu_at(shared_state, fin ? idx - TIMES : idx);
+    const eu_q v = fin ? eu_update<true>(b, fx, fy) : eu_update<false>(b, fx, fy);
+    out[0] = (R)v.r;
+    out[VARS] = (R)v.m;
+    out[2 * VARS] = (R)v.n;
+    out[3 * VARS] = (R)v.e;
 }
 
 __device__ void step(double *shared_state, int idx, int globalTimeStep)
@@ -388,8 +500,8 @@ __device__ __forceinline__ void eu_swap(eu_q &q)
  * evaluated as an x face with the momentum components exchanged in its
  * states and exchanged back in its results; the only operations that then
  * run in another order are commutative (m*n as n*m, m*m + n*n as
- * n*n + m*m), so the values are bitwise those of eu_flux<false> and
- * eu_dissipation<false>, and x and y faces share one instruction stream. */
+ * n*n + m*m), so the values are bitwise those of eu_face_vals<false>, and x
+ * and y faces share one instruction stream. */
 template <class R>
 __device__ __forceinline__ void eu_face(const R *cur, const double *P, double *o, int idx, int stride, bool ydir)
 {
@@ -400,10 +512,8 @@ __device__ __forceinline__ void eu_face(const R *cur, const double *P, double *o
         eu_swap(wq);
         eu_swap(c);
     }
-    const eu_q L = eu_limit(wq, c, pc - pw, pw - pww);
-    const eu_q Rr = eu_limit(c, wq, pc - pw, pe - pc);
-    const eu_rcp rl = eu_recip(L.r), rr = eu_recip(Rr.r);
-    eu_q f = eu_flux<true>(L, Rr, rl, rr), d = eu_dissipation<true>(L, Rr, rl, rr);
+    eu_q f, d;
+    eu_face_vals<true>(wq, c, eu_ratio(pc - pw, eu_recip(pw - pww)), eu_ratio(pc - pw, eu_recip(pe - pc)), f, d);
     if (ydir) {
         eu_swap(f);
         eu_swap(d);
@@ -412,19 +522,16 @@ __device__ __forceinline__ void eu_face(const R *cur, const double *P, double *o
     o[4 * FS] = d.r; o[5 * FS] = d.m; o[6 * FS] = d.n; o[7 * FS] = d.e;
 }
 
-/* 0.5*((((0 + flux_a) + diss_a) - flux_b) - diss_b) per component, face a
- * on the low side of the cell and face b on the high side: the per-cell
- * step's order (eu_divergence) */
+/* ((flux_a + diss_a) - flux_b) - diss_b per component, face a on the low
+ * side of the cell and face b on the high side: the per-cell step's order */
 __device__ __forceinline__ eu_q eu_face_diff(const double *fa, const double *fb)
 {
     constexpr int FS = PS_MAXFACES;
     eu_q a;
-    a.r = 0.0; a.m = 0.0; a.n = 0.0; a.e = 0.0;
-    a.r = a.r + fa[0]; a.m = a.m + fa[FS]; a.n = a.n + fa[2 * FS]; a.e = a.e + fa[3 * FS];
-    a.r = a.r + fa[4 * FS]; a.m = a.m + fa[5 * FS]; a.n = a.n + fa[6 * FS]; a.e = a.e + fa[7 * FS];
-    a.r = a.r - fb[0]; a.m = a.m - fb[FS]; a.n = a.n - fb[2 * FS]; a.e = a.e - fb[3 * FS];
-    a.r = a.r - fb[4 * FS]; a.m = a.m - fb[5 * FS]; a.n = a.n - fb[6 * FS]; a.e = a.e - fb[7 * FS];
-    a.r = a.r * 0.5; a.m = a.m * 0.5; a.n = a.n * 0.5; a.e = a.e * 0.5;
+    a.r = fa[0] + fa[4 * FS] - fb[0] - fb[4 * FS];
+    a.m = fa[FS] + fa[5 * FS] - fb[FS] - fb[5 * FS];
+    a.n = fa[2 * FS] + fa[6 * FS] - fb[2 * FS] - fb[6 * FS];
+    a.e = fa[3 * FS] + fa[7 * FS] - fb[3 * FS] - fb[7 * FS];
     return a;
 }
 
@@ -498,7 +605,6 @@ __device__ __forceinline__ void ps_level(const R *cur, const Prev &prev, R *out,
 
     /* 5. (x and) y divergence and the RK2 update of my cells */
     const bool fin = globalTimeStep % 2 == 0;
-    const double hh = fin ? 1.0 : 0.5;
 #pragma unroll
     for (int m = 0; m < MAXC; ++m) {
         const int t = threadIdx.x + m * PS_NT;
@@ -509,18 +615,8 @@ __device__ __forceinline__ void ps_level(const R *cur, const Prev &prev, R *out,
             const eu_q a = eu_face_diff(fs, fs + 1);
             const int idx = (x0 + i) * SY + (y0 + j);
             const eu_q b = fin ? eu_at(prev, idx) : eu_at(cur, idx);
-            R v[4];
-            if (fin) {
-                v[0] = (R)(b.r + (fx.r * DTDX + a.r * DTDY));
-                v[1] = (R)(b.m + (fx.m * DTDX + a.m * DTDY));
-                v[2] = (R)(b.n + (fx.n * DTDX + a.n * DTDY));
-                v[3] = (R)(b.e + (fx.e * DTDX + a.e * DTDY));
-            } else {
-                v[0] = (R)(b.r + hh * (fx.r * DTDX + a.r * DTDY));
-                v[1] = (R)(b.m + hh * (fx.m * DTDX + a.m * DTDY));
-                v[2] = (R)(b.n + hh * (fx.n * DTDX + a.n * DTDY));
-                v[3] = (R)(b.e + hh * (fx.e * DTDX + a.e * DTDY));
-            }
+            const eu_q u = fin ? eu_update<true>(b, fx, a) : eu_update<false>(b, fx, a);
+            const R v[4] = {(R)u.r, (R)u.m, (R)u.n, (R)u.e};
             if (out) {
                 R *o = out + idx;
                 o[0] = v[0];
@@ -564,31 +660,18 @@ __device__ __forceinline__ void ps_level(const R *cur, const Prev &prev, R *out,
 #define EU_BAND_WOUT (64 - 4 * PS_BAND_H)
 static_assert(EU_BAND_WOUT >= 8, "PS_BAND_H too deep for a 64-column band");
 
-/* face between cells a (low) and b (high) along x (XDIR) or y: pww, pw, pc
- * and pe are the pressures of the cell below a, a, b and the cell above b;
- * flux and dissipation as in eu_face */
-template <bool XDIR>
-__device__ __forceinline__ void eu_face_vals(const eu_q &a, const eu_q &b, double pww, double pw, double pc,
-                                             double pe, eu_q &f, eu_q &d)
+__device__ __forceinline__ eu_rcp eu_lower(const eu_rcp &q)
 {
-    const eu_q L = eu_limit(a, b, pc - pw, pw - pww);
-    const eu_q Rr = eu_limit(b, a, pc - pw, pe - pc);
-    const eu_rcp rl = eu_recip(L.r), rr = eu_recip(Rr.r);
-    f = eu_flux<XDIR>(L, Rr, rl, rr);
-    d = eu_dissipation<XDIR>(L, Rr, rl, rr);
+    eu_rcp o;
+    o.d = ps_from_lower(q.d); o.y = ps_from_lower(q.y);
+    return o;
 }
 
-/* eu_face_diff on values: 0.5*((((0 + fa) + da) - fb) - db) */
-__device__ __forceinline__ eu_q eu_band_diff(const eu_q &fa, const eu_q &da, const eu_q &fb, const eu_q &db)
+__device__ __forceinline__ eu_rcp eu_upper(const eu_rcp &q)
 {
-    eu_q a;
-    a.r = 0.0; a.m = 0.0; a.n = 0.0; a.e = 0.0;
-    a.r = a.r + fa.r; a.m = a.m + fa.m; a.n = a.n + fa.n; a.e = a.e + fa.e;
-    a.r = a.r + da.r; a.m = a.m + da.m; a.n = a.n + da.n; a.e = a.e + da.e;
-    a.r = a.r - fb.r; a.m = a.m - fb.m; a.n = a.n - fb.n; a.e = a.e - fb.e;
-    a.r = a.r - db.r; a.m = a.m - db.m; a.n = a.n - db.n; a.e = a.e - db.e;
-    a.r = a.r * 0.5; a.m = a.m * 0.5; a.n = a.n * 0.5; a.e = a.e * 0.5;
-    return a;
+    eu_rcp o;
+    o.d = ps_from_upper(q.d); o.y = ps_from_upper(q.y);
+    return o;
 }
 
 __device__ __forceinline__ eu_q eu_lower(const eu_q &q)
@@ -617,69 +700,78 @@ struct eu_band_row {
 };
 
 /* The last three rows a level produced (slot tau % 3 holds the newest, so
- * nothing moves between steps), their pressures, and each row's pressure
- * difference to the row before it: the x face (r | r+1) takes
- * p(r+1) - p(r), p(r) - p(r-1) and p(r+2) - p(r+1) as its limiter ratios'
- * numerator and denominators. */
+ * nothing moves between steps), the newest one's pressure, and each row's
+ * pressure difference to the row before it with the reciprocal of that
+ * difference: the x face (r | r+1) takes p(r+1) - p(r) over p(r) - p(r-1)
+ * and over p(r+2) - p(r+1), so each difference divides twice, two steps
+ * apart, and its reciprocal is formed once. */
 template <class R>
 struct eu_band_win {
     eu_band_row<R> q[3];
-    double p[3], dp[3];
+    double p[3];
+    eu_rcp dp[3];
 };
 
-/* (the range check of a valid cell only marks `bad`: the fault flag is
- * written once per wavefront, after the sweep, so that the steps hold no
- * branch) */
+/* Division range of the cells a wavefront met: the extremes of the high
+ * words of rho, E and p (as unsigned integers those of positive numbers are
+ * in the numbers' order, and negative numbers and NaN lie above them all),
+ * and whether a momentum left its range.  The fault flag is written once
+ * per wavefront, after the sweep, so the steps hold no branch. */
+struct eu_band_range {
+    unsigned lo, hi;
+    bool mom;
+    __device__ __forceinline__ void take(const eu_q &q, double p)
+    {
+        const unsigned r = (unsigned)(__double_as_longlong(q.r) >> 32);
+        const unsigned e = (unsigned)(__double_as_longlong(q.e) >> 32);
+        const unsigned k = (unsigned)(__double_as_longlong(p) >> 32);
+        lo = min(min(lo, r), min(e, k));
+        hi = max(max(hi, r), max(e, k));
+        mom |= !(eu_mom_in_range(q.m) & eu_mom_in_range(q.n));
+    }
+    /* 2^-120 has the high word 0x38700000 and 2^120 0x47700000, both with
+     * low word zero; a value in [2^120, 2^120 (1 + 2^-20)) counts as out */
+    __device__ __forceinline__ bool fault() const { return mom | (lo < 0x38700000u) | (hi >= 0x47700000u); }
+};
+
 template <int PH, class R>
-__device__ __forceinline__ void eu_band_push(eu_band_win<R> &w, const eu_band_row<R> &row, bool check, bool &bad)
+__device__ __forceinline__ void eu_band_push(eu_band_win<R> &w, const eu_band_row<R> &row, bool check,
+                                             eu_band_range &rng)
 {
     const eu_q q = row.q();
     const double p = eu_pressure(q);
     w.q[PH] = row;
-    w.dp[PH] = p - w.p[(PH + 2) % 3];
+    w.dp[PH] = eu_recip(p - w.p[(PH + 2) % 3]);
     w.p[PH] = p;
-    bad |= check & !eu_in_range(q.r, q.m, q.n, q.e, p);
+    if (check) rng.take(q, p);
 }
 
 /* Row r of level l from level l-1's window at step phase PH (its newest
  * row, slot PH, is r + 2): the x face (r | r+1), the y faces of row r, the
- * divergences with the x face below (xf, xd, replaced by the new one) and
- * the RK2 update from base (the cell itself, or for a final stage the cell
- * two levels back). */
+ * divergences with the x face below (xc, its flux + dissipation, replaced
+ * by the new one's) and the RK2 update from base (the cell itself, or for a
+ * final stage the cell two levels back).  A lane forms the pressure
+ * difference across its east y face and that difference's reciprocal once
+ * and takes its neighbours' for the two limiter ratios. */
 template <int PH, bool FINAL, class R>
-__device__ __forceinline__ eu_band_row<R> eu_band_cell(const eu_band_win<R> &w, eu_q &xf, eu_q &xd,
-                                                       const eu_q &base2)
+__device__ __forceinline__ eu_band_row<R> eu_band_cell(const eu_band_win<R> &w, eu_q &xc, const eu_q &base2)
 {
     constexpr int pa = (PH + 1) % 3, pb = (PH + 2) % 3;  /* rows r, r + 1 */
     const eu_q a = w.q[pa].q(), b = w.q[pb].q();
     eu_q f, d;
-    {
-        const eu_q L = eu_limit(a, b, w.dp[pb], w.dp[pa]);
-        const eu_q Rr = eu_limit(b, a, w.dp[pb], w.dp[PH]);
-        const eu_rcp rl = eu_recip(L.r), rr = eu_recip(Rr.r);
-        f = eu_flux<true>(L, Rr, rl, rr);
-        d = eu_dissipation<true>(L, Rr, rl, rr);
-    }
-    const double pr = w.p[pa], pu = ps_from_upper(pr);
-    eu_q fe, de;
-    eu_face_vals<false>(a, eu_upper(a), ps_from_lower(pr), pr, pu, ps_from_upper(pu), fe, de);
-    const eu_q fx = eu_band_diff(xf, xd, f, d);
-    const eu_q fy = eu_band_diff(eu_lower(fe), eu_lower(de), fe, de);
-    xf = f;
-    xd = d;
-    const eu_q bs = FINAL ? base2 : a;
+    eu_face_vals<true>(a, b, eu_ratio(w.dp[pb].d, w.dp[pa]), eu_ratio(w.dp[pb].d, w.dp[PH]), f, d);
+    const eu_q ax = eu_less(xc, f, d);
+    xc = eu_sum(f, d);
+    const double pr = w.p[pa];
+    const eu_rcp dy = eu_recip(ps_from_upper(pr) - pr);
+    eu_face_vals<false>(a, eu_upper(a), eu_ratio(dy.d, eu_lower(dy)), eu_ratio(dy.d, eu_upper(dy)), f, d);
+    const eu_q ay = eu_less(eu_lower(eu_sum(f, d)), f, d);
+    const eu_q v = eu_update<FINAL>(FINAL ? base2 : a, ax, ay);
     eu_band_row<R> o;
-    if (FINAL) {
-        o.v[0] = (R)(bs.r + (fx.r * DTDX + fy.r * DTDY));
-        o.v[1] = (R)(bs.m + (fx.m * DTDX + fy.m * DTDY));
-        o.v[2] = (R)(bs.n + (fx.n * DTDX + fy.n * DTDY));
-        o.v[3] = (R)(bs.e + (fx.e * DTDX + fy.e * DTDY));
-    } else {
-        o.v[0] = (R)(bs.r + 0.5 * (fx.r * DTDX + fy.r * DTDY));
-        o.v[1] = (R)(bs.m + 0.5 * (fx.m * DTDX + fy.m * DTDY));
-        o.v[2] = (R)(bs.n + 0.5 * (fx.n * DTDX + fy.n * DTDY));
-        o.v[3] = (R)(bs.e + 0.5 * (fx.e * DTDX + fy.e * DTDY));
-    }
+    o.v[0] = (R)v.r;
+    o.v[1] = (R)v.m;
+    o.v[2] = (R)v.n;
+    o.v[3] = (R)v.e;
     return o;
 }
 
@@ -730,8 +822,8 @@ __device__ __forceinline__ int eu_band_wrap(int r, int nx)
  * compiler may interleave the two levels' independent work. */
 template <int PH, bool FULL, class R>
 __device__ __forceinline__ void eu_band_step(const eu_band_ctx<R> &c, int tau, eu_band_win<R> &w0,
-                                             eu_band_win<R> &w1, eu_q (&xf)[2], eu_q (&xd)[2],
-                                             eu_band_row<R> (&pf)[3], int &lr, bool &bad)
+                                             eu_band_win<R> &w1, eu_q (&xc)[2],
+                                             eu_band_row<R> (&pf)[3], int &lr, eu_band_range &rng)
 {
     /* level A: this step's row (loaded three steps ago) */
     const eu_band_row<R> in = pf[PH];
@@ -743,17 +835,16 @@ __device__ __forceinline__ void eu_band_step(const eu_band_ctx<R> &c, int tau, e
     const int r2 = c.xs + tau - 4;
     const bool two = FULL || (c.hh >= 2 && tau >= 7);
     if (two) eu_band_load(c, eu_band_wrap(r2, c.nx), b2);
-    eu_band_push<PH>(w0, in, true, bad);
+    eu_band_push<PH>(w0, in, true, rng);
     /* level 1 (a half stage), row xs + tau - 2 */
     if (FULL || tau >= 3) {
-        const eu_band_row<R> v1 = eu_band_cell<PH, false>(w0, xf[0], xd[0], eu_q());
-        const bool ok = (FULL || tau >= 4) && c.lane >= 2 && c.lane < 62;
-        eu_band_push<PH>(w1, v1, ok, bad);
-        if (!FULL && ok) eu_band_store(c, 1, c.xs + tau - 2, v1);
+        const eu_band_row<R> v1 = eu_band_cell<PH, false>(w0, xc[0], eu_q());
+        eu_band_push<PH>(w1, v1, FULL || tau >= 4, rng);
+        if (!FULL && tau >= 4) eu_band_store(c, 1, c.xs + tau - 2, v1);
     }
     /* level 2 (the final stage), row xs + tau - 4 */
     if (two) {
-        const eu_band_row<R> v2 = eu_band_cell<PH, true>(w1, xf[1], xd[1], b2.q());
+        const eu_band_row<R> v2 = eu_band_cell<PH, true>(w1, xc[1], b2.q());
         eu_band_store(c, 2, r2, v2);
     }
 }
@@ -790,14 +881,12 @@ __device__ __forceinline__ void ps_band_sweep(R *state, int gts0, int A, const p
     for (int k = 0; k < 3; ++k) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) w0.q[k].v[v] = w1.q[k].v[v] = (R)0;
-        w0.p[k] = w1.p[k] = w0.dp[k] = w1.dp[k] = 0.0;
+        w0.p[k] = w1.p[k] = 0.0;
+        w0.dp[k].d = w1.dp[k].d = w0.dp[k].y = w1.dp[k].y = 0.0;
     }
-    eu_q xf[2], xd[2];
+    eu_q xc[2];
 #pragma unroll
-    for (int l = 0; l < 2; ++l) {
-        xf[l].r = xf[l].m = xf[l].n = xf[l].e = 0.0;
-        xd[l] = xf[l];
-    }
+    for (int l = 0; l < 2; ++l) xc[l].r = xc[l].m = xc[l].n = xc[l].e = 0.0;
     eu_band_row<R> pf[3];
     int lr = eu_band_wrap(c.xs, g.nx);
 #pragma unroll
@@ -806,28 +895,30 @@ __device__ __forceinline__ void ps_band_sweep(R *state, int gts0, int A, const p
         lr = lr + 1 == g.nx ? 0 : lr + 1;
     }
     const int steps = c.rows + 4 * g.hh;
-    bool bad = false;
+    eu_band_range rng = {~0u, 0u, false};
     int tau = 0;
     if (g.hh == 2 && g.wlo == 2) {
         /* warm-up: level 2 starts at step 7, valid cells of level 1 at 4 */
         for (; tau < 9; tau += 3) {
-            eu_band_step<0, false>(c, tau, w0, w1, xf, xd, pf, lr, bad);
-            eu_band_step<1, false>(c, tau + 1, w0, w1, xf, xd, pf, lr, bad);
-            eu_band_step<2, false>(c, tau + 2, w0, w1, xf, xd, pf, lr, bad);
+            eu_band_step<0, false>(c, tau, w0, w1, xc, pf, lr, rng);
+            eu_band_step<1, false>(c, tau + 1, w0, w1, xc, pf, lr, rng);
+            eu_band_step<2, false>(c, tau + 2, w0, w1, xc, pf, lr, rng);
         }
         for (; tau < steps; tau += 3) {
-            eu_band_step<0, true>(c, tau, w0, w1, xf, xd, pf, lr, bad);
-            eu_band_step<1, true>(c, tau + 1, w0, w1, xf, xd, pf, lr, bad);
-            eu_band_step<2, true>(c, tau + 2, w0, w1, xf, xd, pf, lr, bad);
+            eu_band_step<0, true>(c, tau, w0, w1, xc, pf, lr, rng);
+            eu_band_step<1, true>(c, tau + 1, w0, w1, xc, pf, lr, rng);
+            eu_band_step<2, true>(c, tau + 2, w0, w1, xc, pf, lr, rng);
         }
     } else {
         for (; tau < steps; tau += 3) {
-            eu_band_step<0, false>(c, tau, w0, w1, xf, xd, pf, lr, bad);
-            eu_band_step<1, false>(c, tau + 1, w0, w1, xf, xd, pf, lr, bad);
-            eu_band_step<2, false>(c, tau + 2, w0, w1, xf, xd, pf, lr, bad);
+            eu_band_step<0, false>(c, tau, w0, w1, xc, pf, lr, rng);
+            eu_band_step<1, false>(c, tau + 1, w0, w1, xc, pf, lr, rng);
+            eu_band_step<2, false>(c, tau + 2, w0, w1, xc, pf, lr, rng);
         }
     }
-    /* a vector store (a benign race: every writer writes 1) */
-    if (bad) *(volatile int *)&EU_RANGE_FAULT = 1;
+    /* a vector store (a benign race: every writer writes 1).  Level 1 is
+     * valid in lanes 2..61, and what the outer lanes saw of level A is also
+     * seen by the neighbouring bands' inner lanes. */
+    if (rng.fault() && lane >= 2 && lane < 62) *(volatile int *)&EU_RANGE_FAULT = 1;
 }
 #endif /* PS_BAND_COMMON */
