@@ -109,6 +109,9 @@ int ps_memcpy_dtoh(void *dst, const void *src, size_t bytes);
 int ps_memcpy_dtod(void *dst, const void *src, size_t bytes);
 /* Fill bytes (stream ordered). */
 int ps_memset(void *dst, int value, size_t bytes);
+/* Write at most 64 bytes to device memory in stream order without waiting;
+ * the bytes travel as a kernel's argument, so `data` may be reused at once. */
+int ps_write(void *dst, const void *data, size_t bytes);
 
 /* Page-locked host memory: the host side of the asynchronous copies below
  * (no counterpart in the reference, whose copies all wait). */

@@ -124,15 +124,19 @@ def solo_standard_spec(plugin, precision, its, nx, ny):
     return kernels.standard_spec(cu, nv, ops, its, nx, ny, real=real)
 
 
+def solo_swept_spec(plugin, precision, its, b):
+    """The plain swept module of a class."""
+    py, cu64, cu32, nv, ops, _ = PLUGINS[plugin]
+    real = "double" if precision == "fp64" else "float"
+    return kernels.swept_spec(eq_path(cu64 if precision == "fp64" else cu32), nv, ops, its, b, real=real)
+
+
 def solo_specs(plugin, precision, its, b):
     """The plain modules a class uses for a problem running alone: the
     swept phases and the standard modules of the tiles its grids can take
     (a tile no larger than the grid; the tile depends on the grid only
     through that bound)."""
-    py, cu64, cu32, nv, ops, _ = PLUGINS[plugin]
-    real = "double" if precision == "fp64" else "float"
-    cu = eq_path(cu64 if precision == "fp64" else cu32)
-    out = [kernels.swept_spec(cu, nv, ops, its, b, real=real)]
+    out = [solo_swept_spec(plugin, precision, its, b)]
     sides = [s for s in (16, 32, 64, 128, 1 << 16) if s >= b]
     for nx in sides:
         for ny in sides:
@@ -243,7 +247,7 @@ class PluginClass:
         standard kernel with a tile that fits an nx x ny grid), for a
         problem that runs alone."""
         if self._solo is None:
-            sw = solo_specs(self.plugin, self.precision, self.its, self.b)[0]
+            sw = solo_swept_spec(self.plugin, self.precision, self.its, self.b)
             msw = kernels.load(sw)
             self.modules.append(msw)
             self._solo = (sw, msw, {n: msw.get_function(n) for n in kernels.SWEPT_KERNELS})

@@ -192,6 +192,16 @@ __global__ void ps_copy_kernel(double *__restrict__ dst, const double *__restric
     for (; i < n; i += stride) dst[i] = src[i];
 }
 
+struct ps_bytes {
+    unsigned char v[64];
+};
+
+__global__ void ps_write_kernel(unsigned char *dst, ps_bytes b, int n)
+{
+    const int i = threadIdx.x;
+    if (i < n) dst[i] = b.v[i];
+}
+
 // One phase launch: K(state, gts, A0, grid).
 int launch_phase(const ps_swept_plan *p, ps_function f, int gts, int A0, int xoff, int keep_from, int kind)
 {
@@ -594,6 +604,21 @@ int ps_memcpy_dtod_async(void *dst, const void *src, size_t bytes)
 {
     PS_NEED_INIT();
     PS_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, stream()));
+    return 0;
+}
+
+int ps_write(void *dst, const void *data, size_t bytes)
+{
+    PS_NEED_INIT();
+    if (!dst || !data) return fail("ps_write: null address");
+    ps_bytes b = {};
+    if (bytes > sizeof(b.v)) return fail("ps_write: at most 64 bytes");
+    if (bytes == 0) return 0;
+    std::memcpy(b.v, data, bytes);
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(ps_write_kernel, dim3(1), dim3(64), 0, stream(), static_cast<unsigned char *>(dst), b,
+                       static_cast<int>(bytes));
+    PS_HIP(hipGetLastError());
     return 0;
 }
 

@@ -17,8 +17,8 @@ from pysweep_amd import hip, kernels, plugins, schedule
 def range_fault(modules, clear=False):
     """Whether a plugin that checks its division range (the Euler plugin's
     EU_RANGE_FAULT) met a state outside it in any of ``modules`` since the
-    last clear; ``clear`` resets the flags instead (both wait for the work
-    stream).  Modules without the flag never report one."""
+    last clear (waits for the work stream); ``clear`` resets the flags
+    instead, in stream order.  Modules without the flag never report one."""
     hit = False
     for m in modules:
         try:
@@ -26,7 +26,7 @@ def range_fault(modules, clear=False):
         except hip.HipError:
             continue
         if clear:
-            hip.htod(ptr, numpy.zeros(1, numpy.int32))
+            hip.memset_async(ptr, 0, 4)
         else:
             v = numpy.zeros(1, numpy.int32)
             hip.dtoh(v, ptr)
@@ -39,7 +39,9 @@ class _Run:
         self.nv, self.its, self.nx, self.ny, self.T = nv, its, nx, ny, T
         self.dtype = numpy.float64 if real == "double" else numpy.float32
         self.level_bytes = nv * nx * ny * numpy.dtype(self.dtype).itemsize
-        self.ring = hip.DeviceArray(T * self.level_bytes)
+        # the ring, then two records of level sums (sums, sums_async)
+        self._sums_at = -(-T * self.level_bytes // 256) * 256
+        self.ring = hip.DeviceArray(self._sums_at + 2 * hip.SUMS_BYTES)
         self.modules = []
 
     def facade(self):
@@ -54,14 +56,16 @@ class _Run:
         FP64 and in FP32): a debug mode in which a read of a cell that no
         phase wrote -- a skipped private cell, a face outside the sets --
         turns the result into NaN instead of passing unnoticed."""
-        self.ring.fill_bytes(0xFF)
+        self.ring.fill_bytes(0xFF, self.T * self.level_bytes)
 
     def upload_ic(self, ic):
         ic = numpy.ascontiguousarray(ic, dtype=self.dtype)
         if ic.shape != (self.nv, self.nx, self.ny):
             raise ValueError(f"initial condition shape {ic.shape} != {(self.nv, self.nx, self.ny)}")
-        for A in range(self.its):
-            self.ring.upload(ic, (A % self.T) * self.level_bytes)
+        first = self.ring.ptr
+        self.ring.upload(ic)
+        for A in range(1, self.its):  # one copy over the bus; the others stay on the device
+            hip.dtod_async(first + (A % self.T) * self.level_bytes, first, self.level_bytes)
 
     def keep_ic_on_device(self, ic):
         """Device copy of the initial condition for stream-ordered resets."""
@@ -92,8 +96,20 @@ class _Run:
     def sums(self, A):
         """FP64 (sums, sums of magnitudes) of level A's variables, summed on
         the device (for FP32 state too)."""
-        return hip.level_sums(self.ring.ptr + (A % self.T) * self.level_bytes, self.dtype == numpy.float32,
-                              self.nv, self.nx * self.ny)
+        self.sums_async(A, 0)
+        return self.read_sums()[0]
+
+    def sums_async(self, A, record):
+        """Queue the sums of level A into record 0 or 1 (``read_sums``)."""
+        hip.level_sums_async(self.ring.ptr + (A % self.T) * self.level_bytes, self.dtype == numpy.float32, self.nv,
+                             self.nx * self.ny, self.ring.ptr + self._sums_at + record * hip.SUMS_BYTES)
+
+    def read_sums(self):
+        """Both records as (sums, sums of magnitudes) pairs (waits for the
+        work stream)."""
+        n = hip.SUMS_BYTES // 8
+        host = self.ring.download(numpy.empty((2, n)), self._sums_at)
+        return [(h[:self.nv].copy(), h[self.nv:2 * self.nv].copy()) for h in host]
 
     def close(self):
         self.ring.close()

@@ -147,6 +147,7 @@ _swept_run_timed = _sig("ps_swept_run_timed", ctypes.POINTER(SweptPlan), c_int, 
                         ctypes.POINTER(RunStats))
 _standard_run_timed = _sig("ps_standard_run_timed", ctypes.POINTER(StandardPlan), c_int, c_int,
                            ctypes.POINTER(RunStats))
+_write = _sig("ps_write", c_void_p, c_char_p, c_size_t)
 _band_run = _sig("ps_band_run", ctypes.POINTER(BandPlan), c_int, c_int)
 _band_run_timed = _sig("ps_band_run_timed", ctypes.POINTER(BandPlan), c_int, c_int, ctypes.POINTER(RunStats))
 _copy_f64 = _sig("ps_copy_f64", c_void_p, c_void_p, c_size_t)
@@ -166,7 +167,7 @@ EXPORTS = ("ps_version", "ps_last_error", "ps_device_count", "ps_init", "ps_shut
            "ps_compile", "ps_compiler_version",
            "ps_free_host", "ps_module_load", "ps_module_unload", "ps_module_get_global",
            "ps_module_get_function", "ps_function_info", "ps_malloc", "ps_free", "ps_memcpy_htod",
-           "ps_memcpy_dtoh", "ps_memcpy_dtod", "ps_memset", "ps_host_malloc", "ps_host_free",
+           "ps_memcpy_dtoh", "ps_memcpy_dtod", "ps_memset", "ps_write", "ps_host_malloc", "ps_host_free",
            "ps_memcpy_htod_async", "ps_memcpy_dtoh_async", "ps_memcpy_dtod_async", "ps_launch", "ps_synchronize",
            "ps_event_create", "ps_event_record", "ps_event_elapsed_ms", "ps_event_synchronize", "ps_event_query",
            "ps_event_destroy", "ps_stream_wait_event",
@@ -442,6 +443,15 @@ def dtoh(out, dptr):
     return out
 
 
+def write_bytes(dptr, data):
+    """Write a few bytes (at most 64, else as ``htod_bytes``) to device
+    memory in stream order, without waiting: they travel as a kernel's
+    argument."""
+    if len(data) > 64:
+        return htod_bytes(dptr, data)
+    check(_write(dptr, bytes(data), len(data)), "ps_write")
+
+
 def htod_bytes(dptr, data):
     buf = ctypes.create_string_buffer(bytes(data), len(data))
     check(_htod(dptr, ctypes.addressof(buf), len(data)), "ps_memcpy_htod")
@@ -449,6 +459,11 @@ def htod_bytes(dptr, data):
 
 def dtod(dst, src, nbytes):
     check(_dtod(dst, src, nbytes), "ps_memcpy_dtod")
+
+
+def memset_async(dptr, value, nbytes):
+    """Set device memory to a byte value, in stream order."""
+    check(_memset(dptr, int(value) & 0xFF, int(nbytes)), "ps_memset")
 
 
 def synchronize():
@@ -501,6 +516,10 @@ def multi_run(plan, rounds, stats=None):
 def copy_f64(dst, src, n):
     """Stream-ordered device copy of n doubles by the library's copy kernel."""
     check(_copy_f64(dst, src, n), "ps_copy_f64")
+
+
+#: bytes of a level's sums: 2 * nv doubles, nv at most 8
+SUMS_BYTES = 128
 
 
 def level_sums_async(level_ptr, fp32, nv, cells, out_ptr):

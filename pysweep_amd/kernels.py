@@ -9,6 +9,8 @@ import dataclasses
 import os
 import re
 
+import numpy
+
 from pysweep_amd import compiler
 from pysweep_amd.equations import path as eq_path
 
@@ -268,15 +270,16 @@ def band_rows(spec, nx, ny, simds=BAND_SIMDS):
     wout = band_out_columns(spec)
     bands = -(-ny // wout)
     work_of = band_wave_work(spec)
-    best = None
-    for rows in range(min(4, nx), min(nx, 256) + 1):
-        waves = bands * -(-nx // rows)
-        work = work_of(rows)
-        m = -(-waves // simds)
-        cost = work / 0.815 if m == 1 else m * work
-        if best is None or cost <= best[0]:
-            best = (cost, rows)
-    return best[1]
+    # segments of 4 rows (or the grid's) to 256; of the segments that a
+    # wavefront works equally long on (its steps are rounded up to 3) only the
+    # longest
+    rows = numpy.arange(min(4, nx), min(nx, 256) + 1)
+    work = work_of(rows)
+    rows = rows[numpy.append(work[1:] != work[:-1], True)]
+    work = work_of(rows)
+    m = -(-bands * -(-nx // rows) // simds)
+    cost = numpy.where(m == 1, work / 0.815, m * work)
+    return int(rows[len(cost) - 1 - int(numpy.argmin(cost[::-1]))])  # the longest of the cheapest
 
 
 def band_wave_work(spec):
@@ -284,15 +287,15 @@ def band_wave_work(spec):
     sweep steps (each computing every level of the launch for one row): the
     segment plus the launch's x halo, rounded up to the step loop's
     unrolling (3); level l computes from the step its first valid row appears
-    on; a few steps' worth of set-up is added."""
+    on; a few steps' worth of set-up is added.  (Rows: a number or an array.)"""
     H, k = spec.levels, spec.ops
     point = has_point_update(spec.user_path)
 
     def work(rows):
         steps = 3 * -(-(rows + 2 * k * H) // 3)
         if point:
-            return sum(steps - 2 * l for l in range(1, H + 1)) + 2 * H
-        return sum(steps - (2 * k * l - 1) for l in range(1, H + 1)) + 4
+            return H * steps - H * (H + 1) + 2 * H
+        return H * steps - k * H * (H + 1) + H + 4
     return work
 
 
@@ -313,7 +316,6 @@ def band_multi_rows(spec, shapes, simds=BAND_SIMDS):
     issues about 0.815 of the time.  Measured on MI355X (the 256 Euler problems of
     the 512-problem mix, engine seconds by cap): 24 0.940, 32 0.916, 48
     0.894, 64 0.866, 96 0.849 (chosen), 128 0.855, 192 0.861, 256 0.908."""
-    import numpy
     if not shapes:
         return []
     wout = band_out_columns(spec)
@@ -321,7 +323,7 @@ def band_multi_rows(spec, shapes, simds=BAND_SIMDS):
     nx = numpy.array([s[0] for s in shapes], dtype=numpy.int64)
     bands = -(-numpy.array([s[1] for s in shapes], dtype=numpy.int64) // wout)
     top = BAND_MULTI_CAPS[-1]
-    table = numpy.array([0] + [work_of(r) for r in range(1, top + 1)], dtype=numpy.int64)
+    table = work_of(numpy.arange(top + 1, dtype=numpy.int64))
     best = None
     for cap in BAND_MULTI_CAPS:
         segs = -(-nx // cap)
@@ -369,6 +371,8 @@ def swept_faces(b, ops):
     return (m + 1) * m
 
 
+_SCRATCH = {}  # absolute path -> (source text it was read from, level_scratch's answer)
+
 _SCRATCH_RE = re.compile(r"^[ \t]*#[ \t]*define[ \t]+PS_LEVEL_SCRATCH\((\w+),\s*(\w+)\)(.*)$", re.M)
 
 
@@ -377,7 +381,15 @@ def level_scratch(user_path):
     (doubles of LDS scratch), or None without a level update."""
     if not has_level_update(user_path):
         return None
-    m = _SCRATCH_RE.search(read_plugin_source(user_path))
+    text, key = read_plugin_source(user_path), os.path.abspath(user_path)
+    hit = _SCRATCH.get(key)
+    if hit is None or hit[0] is not text:
+        hit = _SCRATCH[key] = (text, _read_level_scratch(text))
+    return hit[1]
+
+
+def _read_level_scratch(text):
+    m = _SCRATCH_RE.search(text)
     if m is None:
         return lambda cells, faces: 0
     a, b, expr = m.group(1), m.group(2), m.group(3).strip()
@@ -390,8 +402,7 @@ def level_scratch(user_path):
 def level_update_in_standard(user_path):
     """False when the plugin asks the standard kernel to keep its per-cell
     step (PS_LEVEL_SWEPT_ONLY)."""
-    return re.search(r"^[ \t]*#[ \t]*define[ \t]+PS_LEVEL_SWEPT_ONLY\b", read_plugin_source(user_path),
-                     re.M) is None
+    return not _defines_macro(user_path, "PS_LEVEL_SWEPT_ONLY")
 
 
 def level_in_place(user_path, generic=False):
@@ -400,8 +411,7 @@ def level_in_place(user_path, generic=False):
     writing it), so a swept window of ITS levels suffices."""
     if generic or not has_level_update(user_path):
         return False
-    return re.search(r"^[ \t]*#[ \t]*define[ \t]+PS_LEVEL_INPLACE\b", read_plugin_source(user_path),
-                     re.M) is not None
+    return _defines_macro(user_path, "PS_LEVEL_INPLACE")
 
 
 def min_slots(user_path, its, generic=False):

@@ -78,7 +78,7 @@ class _Driver:
             for ptr, n in dst.copies:
                 if len(data) > n:
                     raise ValueError(f"{len(data)} bytes do not fit device global {dst.name!r} ({n} bytes)")
-                _hip().htod_bytes(ptr, data)
+                _hip().write_bytes(ptr, data)
         else:
             _hip().htod_bytes(int(dst), data)
 

@@ -248,7 +248,7 @@ class Solver(object):
 
     def _setup_device(self):
         nv, nx, ny = self.initialConditions.shape
-        self._sums0 = None
+        self._sums0 = False
         t = dict(self.tuning)
         if self.simulation and self.share < 1:
             # CPU/GPU split (core/process.py:81-176): block rows divided by share
@@ -298,8 +298,10 @@ class Solver(object):
             self._run.poison()
         self._run.upload_ic(self.initialConditions)
         self._run.range_fault(clear=True)
-        # FP64 sums of the conserved quantities at the start (device-side)
-        self._sums0 = self._run.sums(self.intermediate - 1)
+        # FP64 sums of the conserved quantities at the start (device-side;
+        # read with the final level's)
+        self._run.sums_async(self.intermediate - 1, 0)
+        self._sums0 = True
 
     def _collector(self):
         s = self.intermediate
@@ -323,12 +325,13 @@ class Solver(object):
         self.result = self._run.level(last_full)
         self.result_step = (last_full - (s - 1)) // s
         self.result_level = self.final_level
-        self.final_state = self._run.level(self.final_level)
+        self.final_state = self.result.copy() if last_full == self.final_level else self._run.level(self.final_level)
         # the final level's conserved sums against the initial ones (GPU-only runs)
         self.conservation = None
-        if getattr(self, "_sums0", None) is not None:
+        if getattr(self, "_sums0", False):
             from pysweep_amd import device
-            self.conservation = device.conservation(self._sums0, self._run.sums(self.final_level))
+            self._run.sums_async(self.final_level, 1)
+            self.conservation = device.conservation(*self._run.read_sums())
         full_steps = self.stages / s
         nv, nx, ny = self.globalShape
         self.gcups = nx * ny * full_steps / self.solve_seconds / 1e9 if self.solve_seconds else None
