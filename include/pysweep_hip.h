@@ -266,9 +266,10 @@ typedef struct ps_band_grid {
     int T;          /* ring levels                                         */
     int hh;         /* levels of this launch                               */
     int wlo;        /* levels hh' >= wlo of the launch are written         */
-    int rows;       /* output rows per wavefront                           */
+    int rows;       /* output rows per wavefront (per chain, with chains)  */
     int bands;      /* ceil(ny / (128 - 2 * levels))                       */
     int segs;       /* ceil(nx / rows)                                     */
+    int chain;      /* 0, or the wavefronts of a chain                     */
 } ps_band_grid;
 
 typedef struct ps_band_plan {
@@ -281,9 +282,13 @@ typedef struct ps_band_plan {
     int wout;       /* output columns per band (the kernel's band width less
                        its halo columns: 128 - 2*levels for a point-update
                        plugin, 64 - 2*k*levels for a plugin sweep)          */
-    int rows;       /* output rows per wavefront (> 0)                     */
+    int rows;       /* output rows per wavefront, or per chain (> 0)       */
     int store_all;  /* 1: write every level; 0: the last s of each launch  */
     ps_function band;
+    int chain;      /* 0: wavefronts work by themselves; 4: a workgroup's
+                       four wavefronts share `rows` rows and exchange their
+                       segments' edges (a plugin sweep with
+                       PS_HAS_BAND_CHAIN)                                  */
 } ps_band_plan;
 
 /* Run stages from absolute level A (which must be complete in the ring and

@@ -967,8 +967,8 @@ class Engine:
                 if g0 < g1:
                     spec = band[0]
                     bplan = hip.BandPlan(state=t.ring.ptr, nx=t.nx, ny=t.ny, its=cls.its, T=T, levels=spec.levels,
-                                         wout=kernels.band_out_columns(spec),
-                                         rows=kernels.band_rows(spec, t.nx, t.ny), store_all=0, band=band[2])
+                                         wout=kernels.band_out_columns(spec), store_all=0, band=band[2],
+                                         **kernels.band_launch(spec, t.nx, t.ny)[1])
                     hip.band_run(bplan, cls.its - 2 + g0, g1 - g0)
                     self.band_stages += g1 - g0
             else:

@@ -804,6 +804,7 @@ static int band_run(const ps_band_plan *p, int A, int stages)
     if (stages < 0) return fail("band solve: negative stage count");
     const int wout = p->wout;
     if (wout < 1 || wout > 128) return fail("band solve: output columns per band must be 1..128");
+    if (p->chain != 0 && p->chain != 4) return fail("band solve: a chain has 4 wavefronts (0: no chains)");
     ps_band_grid g;
     g.nx = p->nx;
     g.ny = p->ny;
@@ -811,9 +812,10 @@ static int band_run(const ps_band_plan *p, int A, int stages)
     g.rows = p->rows;
     g.bands = (p->ny + wout - 1) / wout;
     g.segs = (p->nx + p->rows - 1) / p->rows;
-    const long long waves = static_cast<long long>(g.bands) * g.segs;
-    if (waves > (1LL << 30)) return fail("band solve: grid too large");
-    const unsigned groups = static_cast<unsigned>((waves + 3) / 4);
+    g.chain = p->chain;
+    const long long parts = static_cast<long long>(g.bands) * g.segs;  // wavefronts, or chains
+    if (parts > (1LL << 30)) return fail("band solve: grid too large");
+    const unsigned groups = static_cast<unsigned>(g.chain ? parts : (parts + 3) / 4);
     void *state = p->state;
     for (int done = 0; done < stages;) {
         g.hh = stages - done < H ? stages - done : H;

@@ -244,12 +244,12 @@ class BandRun(_Run):
         super().__init__(nv, its, nx, ny, self.spec.levels + its, real)
         mod = kernels.load(self.spec)
         self.modules = [mod]
-        self.rows = int(rows or kernels.band_rows(self.spec, nx, ny))
-        if self.rows < 1:
+        if rows is not None and int(rows) < 1:
             raise ValueError("band rows must be positive")
+        self.rows, shape = kernels.band_launch(self.spec, nx, ny, rows)
         self.plan = hip.BandPlan(state=self.ring.ptr, nx=nx, ny=ny, its=its, T=self.T, levels=self.spec.levels,
-                                 wout=kernels.band_out_columns(self.spec), rows=self.rows, store_all=0,
-                                 band=mod.get_function("Band"))
+                                 wout=kernels.band_out_columns(self.spec), store_all=0,
+                                 band=mod.get_function("Band"), **shape)
 
     def run(self, times, on_level=None, stats=None):
         """The ``times.stages + times.tail`` stages of a swept schedule

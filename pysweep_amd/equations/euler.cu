@@ -633,30 +633,50 @@ __device__ __forceinline__ void ps_level(const R *cur, const Prev &prev, R *out,
 /*
  * Band sweep (PS_HAS_BAND): the swept solve's kernel with every level of a
  * launch in registers.  One wavefront owns a band of 64 columns, one column
- * per lane, and sweeps it along x; a launch of PS_BAND_H stages reads level
- * A over the band and writes level A + PS_BAND_H over its middle
- * 64 - 4 * PS_BAND_H columns (the radius-2 stencil costs two halo columns
- * per level on each side, recomputed by the neighbouring bands instead of
- * exchanged).
+ * per lane, and a segment of rows, and sweeps it along x; a launch of
+ * PS_BAND_H = 2 stages (one RK2 step) reads level A over the band and writes
+ * level A + 2 over its middle 64 - 4 * PS_BAND_H columns (the radius-2
+ * stencil costs two halo columns per level on each side, recomputed by the
+ * neighbouring bands instead of exchanged).
  *
- * Step tau brings in row xs + tau of level A (xs = x0 - 2 * hh) and, for
- * l = 1..hh in order, computes row xs + tau - 2 * l of level A + l.  Each
- * level keeps the last five rows it produced (states, in the storage type)
- * and the last four rows' pressures: the x face between rows r and r + 1
- * needs the pressures of rows r - 1 .. r + 2 and the states of r and r + 1,
- * and a final RK2 stage needs its cell two levels back, four rows behind.
- * The x face below a row is the one above the row before, carried from the
- * previous step; the y face east of a column is computed by its lane from
- * the neighbouring lanes' states and pressures (DPP), and the west one is
- * the lower lane's east face.  Every face, pressure and update is evaluated
- * by the functions and in the order of ps_level and the per-cell step, so
- * results are bitwise theirs.  Rows and columns that a level cannot yet
- * compute correctly (warm-up steps, the outermost lanes) hold garbage that
- * no valid cell ever reads; only valid cells are range-checked and stored.
- * Launches start on full steps (the first stage of a launch never reads
- * the level two back).
+ * A segment is sheared along x: the wavefront of rows [a, a + n) computes
+ * rows [a + 2, a + n + 2) of level A + 1 and [a + 4, a + n + 4) of level
+ * A + 2.  Its first rows then need no halo (level A is in memory), and at its
+ * end level A + 2 lacks the first four level A + 1 rows of the segment after
+ * it, a + n + 2 .. a + n + 5.  In a chain (PS_HAS_BAND_CHAIN: the wavefronts
+ * of one workgroup on consecutive segments of a band) that segment's
+ * wavefront computed them at its own start and left them in LDS; the chain's
+ * last wavefront, and every wavefront of a launch without chains, computes
+ * them itself.  Of the rows a segment recomputed at both ends (two and a
+ * face on each side) a chain of four keeps a quarter, which is what small
+ * segments are made of: Euler 1024^2 has 19 bands, so that 2048 wavefronts
+ * are segments of ten rows.
+ *
+ * Step tau brings in row a + tau of level A and computes row a + tau - 2 l
+ * of level A + l.  Each level keeps the last three rows it produced (states,
+ * in the storage type) and their pressure differences: the x face between
+ * rows r and r + 1 needs the pressures of rows r - 1 .. r + 2 and the states
+ * of r and r + 1.  The x face below a row is the one above the row before,
+ * carried from the previous step; the y face east of a column is computed
+ * by its lane from the neighbouring lanes' states and pressure differences
+ * (DPP), and the west one is the lower lane's east face.  Every face,
+ * pressure and update is evaluated by the functions and in the order of
+ * ps_level and the per-cell step, so results are bitwise theirs.  Rows and
+ * columns that a level cannot yet compute correctly (first steps, the
+ * outermost lanes) hold garbage that no valid cell ever reads; only valid
+ * cells are range-checked and stored.  Launches start on full steps (the
+ * first stage of a launch never reads the level two back).
  */
 #define PS_HAS_BAND 1
+#define PS_HAS_BAND_CHAIN 1
+/* fewest rows of a chain's wavefronts (the rows left in LDS at steps 4..7 are
+ * read from step n + 4 on, after the barrier behind step 8), and the rows the
+ * last one takes less for computing four level-1 rows more */
+#define PS_BAND_MIN_ROWS 5
+#define PS_BAND_LAST_LESS 2
+/* two wavefronts per SIMD (256 VGPRs): left to itself the compiler takes more
+ * registers and one wavefront */
+#define PS_BAND_OCC __attribute__((amdgpu_waves_per_eu(2)))
 #define EU_BAND_WOUT (64 - 4 * PS_BAND_H)
 static_assert(EU_BAND_WOUT >= 8, "PS_BAND_H too deep for a 64-column band");
 
@@ -775,6 +795,17 @@ __device__ __forceinline__ eu_band_row<R> eu_band_cell(const eu_band_win<R> &w, 
     return o;
 }
 
+/* the x face (r | r+1) alone: the one below a segment's first row */
+template <int PH, class R>
+__device__ __forceinline__ void eu_band_xface(const eu_band_win<R> &w, eu_q &xc)
+{
+    constexpr int pa = (PH + 1) % 3, pb = (PH + 2) % 3;
+    eu_q f, d;
+    eu_face_vals<true>(w.q[pa].q(), w.q[pb].q(), eu_ratio(w.dp[pb].d, w.dp[pa]), eu_ratio(w.dp[pb].d, w.dp[PH]), f,
+                       d);
+    xc = eu_sum(f, d);
+}
+
 #define EU_GLOBAL __attribute__((address_space(1)))
 
 template <class R>
@@ -785,26 +816,49 @@ struct eu_band_ctx {
     EU_GLOBAL R *state;
     const EU_GLOBAL R *in;  /* level A */
     size_t cells;
-    int s0, T, nx, ny, wlo, hh, x0, rows, xs, col, oc, lane;
+    int s0, T, nx, ny, wlo, hh;
+    int n, e1;         /* rows of the segment; level 1 is computed until step e1 */
+    unsigned col, oc;  /* this lane's column in bytes; the same unwrapped */
     bool out_col;
 };
+
+/* Rows are the same in every lane, so a row's address is scalar and a
+ * lane's column a 32-bit offset that the load or store adds by itself.  The
+ * empty asm statements keep it so: the compiler would carry the column as a
+ * 64-bit number around the loop and add every row to it in vector
+ * instructions, 6 a cell. */
+__device__ __forceinline__ unsigned eu_band_lane(unsigned bytes)
+{
+    unsigned o;
+    asm volatile("" : "=v"(o) : "0"(bytes));
+    return o;
+}
+
+template <class T>
+__device__ __forceinline__ T *eu_band_at(T *row, unsigned bytes)
+{
+    typedef EU_GLOBAL char B;
+    asm("" : "+s"(row));
+    return (T *)((B *)(row) + bytes);
+}
 
 template <class R>
 __device__ __forceinline__ void eu_band_load(const eu_band_ctx<R> &c, int row, eu_band_row<R> &o)
 {
-    const EU_GLOBAL R *p = c.in + (size_t)row * c.ny + c.col;
+    const unsigned col = eu_band_lane(c.col);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) o.v[v] = p[v * c.cells];
+    for (int v = 0; v < 4; ++v) o.v[v] = *eu_band_at(c.in + (v * c.cells + (size_t)row * c.ny), col);
 }
 
 template <class R>
 __device__ __forceinline__ void eu_band_store(const eu_band_ctx<R> &c, int l, int row, const eu_band_row<R> &o)
 {
-    if (l >= c.wlo && c.out_col && row >= c.x0 && row < c.x0 + c.rows) {
-        const int slot = c.s0 + l >= c.T ? c.s0 + l - c.T : c.s0 + l;
-        EU_GLOBAL R *dst = c.state + (size_t)slot * NV * c.cells + (size_t)row * c.ny + c.oc;
+    const int slot = c.s0 + l >= c.T ? c.s0 + l - c.T : c.s0 + l;
+    if (c.out_col) {
+        const unsigned col = eu_band_lane(c.oc);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) dst[v * c.cells] = o.v[v];
+        for (int v = 0; v < 4; ++v)
+            *eu_band_at(c.state + (((size_t)slot * NV + v) * c.cells + (size_t)row * c.ny), col) = o.v[v];
     }
 }
 
@@ -816,46 +870,80 @@ __device__ __forceinline__ int eu_band_wrap(int r, int nx)
     return r < 0 ? r + nx : r;
 }
 
-/* One step (phase PH = tau % 3) of a one-step (two-stage) launch.  FULL:
- * a step of the steady state of a two-level launch that writes level 2
- * only (both levels valid; no test until the final store), so that the
- * compiler may interleave the two levels' independent work. */
+__device__ __forceinline__ int eu_band_next(int r, int nx) { return r + 1 == nx ? 0 : r + 1; }
+
+/* rows a level reads, loads and stores next (wrapped) */
+struct eu_band_rows {
+    int load;   /* level A, three steps ahead             */
+    int out1;   /* level A + 1's row of this step          */
+    int out2;   /* level A + 2's, and its base in level A  */
+};
+
+/* One step (phase PH = tau % 3) of a one-step (two-stage) launch.  FULL: a
+ * step of the steady state of a two-level launch that writes level 2 only
+ * (both levels valid; no test), so that the compiler may interleave the two
+ * levels' independent work.  pub: where this wavefront leaves its first four
+ * level-1 rows (or null); nxt: where the next segment's lie (or null). */
 template <int PH, bool FULL, class R>
 __device__ __forceinline__ void eu_band_step(const eu_band_ctx<R> &c, int tau, eu_band_win<R> &w0,
-                                             eu_band_win<R> &w1, eu_q (&xc)[2],
-                                             eu_band_row<R> (&pf)[3], int &lr, eu_band_range &rng)
+                                             eu_band_win<R> &w1, eu_q (&xc)[2], eu_band_row<R> (&pf)[3],
+                                             eu_band_rows &r, eu_band_range &rng, R *pub, const R *nxt)
 {
-    /* level A: this step's row (loaded three steps ago) */
-    const eu_band_row<R> in = pf[PH];
-    eu_band_load(c, lr, pf[PH]);
-    lr = lr + 1 == c.nx ? 0 : lr + 1;
+    const int lane = threadIdx.x & 63;
     /* the base of the final stage: level A two rows behind level 1's row,
      * re-read (this wavefront loaded it four steps ago) */
     eu_band_row<R> b2;
-    const int r2 = c.xs + tau - 4;
-    const bool two = FULL || (c.hh >= 2 && tau >= 7);
-    if (two) eu_band_load(c, eu_band_wrap(r2, c.nx), b2);
-    eu_band_push<PH>(w0, in, true, rng);
-    /* level 1 (a half stage), row xs + tau - 2 */
-    if (FULL || tau >= 3) {
-        const eu_band_row<R> v1 = eu_band_cell<PH, false>(w0, xc[0], eu_q());
-        eu_band_push<PH>(w1, v1, FULL || tau >= 4, rng);
-        if (!FULL && tau >= 4) eu_band_store(c, 1, c.xs + tau - 2, v1);
+    const bool two = FULL || (c.hh >= 2 && tau >= 8 && tau < c.n + 8);
+    if (FULL || tau < c.e1) {
+        /* level A: this step's row (loaded three steps ago) */
+        const eu_band_row<R> in = pf[PH];
+        eu_band_load(c, r.load, pf[PH]);
+        r.load = eu_band_next(r.load, c.nx);
+        if (two) eu_band_load(c, r.out2, b2);
+        eu_band_push<PH>(w0, in, true, rng);
+        if (!FULL && PH == 0 && tau == 3) {  /* the face below the segment's first row */
+            eu_band_xface<PH>(w0, xc[0]);
+        } else if (FULL || tau >= 4) {
+            /* level 1 (a half stage) */
+            const eu_band_row<R> v1 = eu_band_cell<PH, false>(w0, xc[0], eu_q());
+            eu_band_push<PH>(w1, v1, true, rng);
+            if (!FULL) {
+                if (pub && tau < 8)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) pub[((tau - 4) * 4 + v) * 64 + lane] = v1.v[v];
+                if (c.wlo <= 1 && tau < c.n + 4) eu_band_store(c, 1, r.out1, v1);
+            }
+        }
+    } else {
+        if (two) eu_band_load(c, r.out2, b2);
+        if (nxt && tau < c.n + 8) {
+            eu_band_row<R> v1;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) v1.v[v] = nxt[((tau - c.n - 4) * 4 + v) * 64 + lane];
+            eu_band_push<PH>(w1, v1, false, rng);
+        }
     }
-    /* level 2 (the final stage), row xs + tau - 4 */
-    if (two) {
+    /* level 2 (the final stage) */
+    if (!FULL && PH == 1 && tau == 7) {
+        eu_band_xface<PH>(w1, xc[1]);
+    } else if (two) {
         const eu_band_row<R> v2 = eu_band_cell<PH, true>(w1, xc[1], b2.q());
-        eu_band_store(c, 2, r2, v2);
+        eu_band_store(c, 2, r.out2, v2);
     }
+    r.out1 = eu_band_next(r.out1, c.nx);
+    r.out2 = eu_band_next(r.out2, c.nx);
 }
 
-template <class R>
-__device__ __forceinline__ void ps_band_sweep(R *state, int gts0, int A, const ps_band_grid &g, int band, int seg)
+/* The segment of rows [a, a + n) of band `band`; CHAIN: the workgroup's
+ * wavefronts are a chain and meet at one barrier (every wavefront of the
+ * workgroup passes it). */
+template <bool CHAIN, class R>
+__device__ __forceinline__ void eu_band_segment(R *state, int A, const ps_band_grid &g, int band, int a, int n,
+                                                R *pub, const R *nxt)
 {
     static_assert(PS_BAND_H == 2, "the Euler band sweep takes one RK2 step (two stages) per launch");
     constexpr int WOUT = EU_BAND_WOUT;
     const int lane = threadIdx.x & 63;
-    (void)gts0;  /* launches start on full steps: level 1 is a half stage, level 2 a final one */
     eu_band_ctx<R> c;
     c.state = (EU_GLOBAL R *)state;  /* device memory */
     c.cells = (size_t)g.nx * g.ny;
@@ -866,15 +954,13 @@ __device__ __forceinline__ void ps_band_sweep(R *state, int gts0, int A, const p
     c.in = c.state + (size_t)c.s0 * NV * c.cells;
     c.hh = g.hh;
     c.wlo = g.wlo;
-    c.x0 = seg * g.rows;
-    c.rows = min(g.rows, g.nx - c.x0);
-    c.xs = c.x0 - 2 * g.hh;
-    c.lane = lane;
+    c.n = n;
+    c.e1 = n + (g.hh >= 2 && !nxt ? 8 : 4);
     const int o = lane - 2 * PS_BAND_H;  /* band-local output column */
-    c.oc = band * WOUT + o;
-    c.col = eu_band_wrap(c.oc, g.ny);
-    c.out_col = o >= 0 && o < WOUT && c.oc < g.ny;
-    /* defined values in what the warm-up steps read before any level has
+    c.out_col = o >= 0 && o < WOUT && band * WOUT + o < g.ny;
+    c.oc = (unsigned)(band * WOUT + o) * (unsigned)sizeof(R);
+    c.col = (unsigned)eu_band_wrap(band * WOUT + o, g.ny) * (unsigned)sizeof(R);
+    /* defined values in what the first steps read before any level has
      * produced it (never used by a valid cell) */
     eu_band_win<R> w0, w1;
 #pragma unroll
@@ -887,38 +973,62 @@ __device__ __forceinline__ void ps_band_sweep(R *state, int gts0, int A, const p
     eu_q xc[2];
 #pragma unroll
     for (int l = 0; l < 2; ++l) xc[l].r = xc[l].m = xc[l].n = xc[l].e = 0.0;
+    eu_band_rows r;
+    r.load = eu_band_wrap(a, g.nx);
+    r.out1 = eu_band_wrap(a - 2, g.nx);
+    r.out2 = eu_band_wrap(a - 4, g.nx);
     eu_band_row<R> pf[3];
-    int lr = eu_band_wrap(c.xs, g.nx);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        eu_band_load(c, lr, pf[k]);
-        lr = lr + 1 == g.nx ? 0 : lr + 1;
+        eu_band_load(c, r.load, pf[k]);
+        r.load = eu_band_next(r.load, g.nx);
     }
-    const int steps = c.rows + 4 * g.hh;
+    const int steps = n + (g.hh >= 2 ? 8 : 4);
+    const int full = g.hh == 2 && g.wlo == 2 ? min(c.e1, n + 8) : 0;  /* end of the steady state */
     eu_band_range rng = {~0u, 0u, false};
     int tau = 0;
-    if (g.hh == 2 && g.wlo == 2) {
-        /* warm-up: level 2 starts at step 7, valid cells of level 1 at 4 */
-        for (; tau < 9; tau += 3) {
-            eu_band_step<0, false>(c, tau, w0, w1, xc, pf, lr, rng);
-            eu_band_step<1, false>(c, tau + 1, w0, w1, xc, pf, lr, rng);
-            eu_band_step<2, false>(c, tau + 2, w0, w1, xc, pf, lr, rng);
-        }
-        for (; tau < steps; tau += 3) {
-            eu_band_step<0, true>(c, tau, w0, w1, xc, pf, lr, rng);
-            eu_band_step<1, true>(c, tau + 1, w0, w1, xc, pf, lr, rng);
-            eu_band_step<2, true>(c, tau + 2, w0, w1, xc, pf, lr, rng);
-        }
-    } else {
-        for (; tau < steps; tau += 3) {
-            eu_band_step<0, false>(c, tau, w0, w1, xc, pf, lr, rng);
-            eu_band_step<1, false>(c, tau + 1, w0, w1, xc, pf, lr, rng);
-            eu_band_step<2, false>(c, tau + 2, w0, w1, xc, pf, lr, rng);
-        }
+    for (; tau < 9 || (tau < steps && full == 0); tau += 3) {
+        eu_band_step<0, false>(c, tau, w0, w1, xc, pf, r, rng, pub, nxt);
+        eu_band_step<1, false>(c, tau + 1, w0, w1, xc, pf, r, rng, pub, nxt);
+        eu_band_step<2, false>(c, tau + 2, w0, w1, xc, pf, r, rng, pub, nxt);
+        if (CHAIN && tau == 6) __syncthreads();
+    }
+    for (; tau + 3 <= full; tau += 3) {
+        eu_band_step<0, true>(c, tau, w0, w1, xc, pf, r, rng, pub, nxt);
+        eu_band_step<1, true>(c, tau + 1, w0, w1, xc, pf, r, rng, pub, nxt);
+        eu_band_step<2, true>(c, tau + 2, w0, w1, xc, pf, r, rng, pub, nxt);
+    }
+    for (; tau < steps; tau += 3) {
+        eu_band_step<0, false>(c, tau, w0, w1, xc, pf, r, rng, pub, nxt);
+        eu_band_step<1, false>(c, tau + 1, w0, w1, xc, pf, r, rng, pub, nxt);
+        eu_band_step<2, false>(c, tau + 2, w0, w1, xc, pf, r, rng, pub, nxt);
     }
     /* a vector store (a benign race: every writer writes 1).  Level 1 is
      * valid in lanes 2..61, and what the outer lanes saw of level A is also
      * seen by the neighbouring bands' inner lanes. */
     if (rng.fault() && lane >= 2 && lane < 62) *(volatile int *)&EU_RANGE_FAULT = 1;
+}
+
+/* one wavefront's segment by itself */
+template <class R>
+__device__ __forceinline__ void ps_band_sweep(R *state, int gts0, int A, const ps_band_grid &g, int band, int seg)
+{
+    (void)gts0;  /* launches start on full steps: level 1 is a half stage, level 2 a final one */
+    const int a = seg * g.rows;
+    eu_band_segment<false>(state, A, g, band, a, min(g.rows, g.nx - a), static_cast<R *>(nullptr),
+                           static_cast<const R *>(nullptr));
+}
+
+/* rows that a chain's wavefronts leave for the one before (PS_BAND_CHAIN
+ * wavefronts: each but the first leaves 4 rows of 4 variables) */
+#define PS_BAND_CHAIN_WORDS (4 * 4 * 64)
+
+/* wavefront k of a chain: rows [a, a + n), `last` if no wavefront follows */
+template <class R>
+__device__ __forceinline__ void ps_band_sweep_chain(R *state, int gts0, int A, const ps_band_grid &g, int band,
+                                                    int a, int n, R *pub, const R *nxt)
+{
+    (void)gts0;
+    eu_band_segment<true>(state, A, g, band, a, n, pub, nxt);
 }
 #endif /* PS_BAND_COMMON */

@@ -211,16 +211,18 @@ def band_multi_levels(user_path, its, real="double"):
 
 #: cells from which a plugin's own band sweep (Euler: one column per lane,
 #: a 2-column halo per level) is the faster swept kernel: its 64-column
-#: bands leave small grids too few wavefronts.  Measured on MI355X (Euler,
-#: GCUPS, band / phase kernels b=16): 128^2 0.67 / 0.83, 256^2 2.64 / 3.20,
-#: 384^2 5.81 / 4.82, 512^2 7.55 / 7.52, 1024^2 14.41 / 9.73.  Heat's band
-#: kernel led at every size measured (64^2 to 8192^2).
+#: bands leave small grids too few wavefronts.  Measured on MI355X when the
+#: line was drawn (Euler, GCUPS, band / phase kernels b=16): 128^2 0.67 /
+#: 0.83, 256^2 2.64 / 3.20, 384^2 5.81 / 4.82, 1024^2 14.41 / 9.73; now (us a
+#: step) 256^2 15.6 / 18.7, 384^2 18.7 / 27.5, 1024^2 56.6 / 96.  Heat's
+#: band kernel led at every size measured (64^2 to 8192^2).
 BAND_SWEEP_MIN_CELLS = 1 << 17
-#: cells from which the Euler band sweep outruns the standard kernel
-#: (GCUPS, band / standard: 512^2 7.60 / 10.22, 768^2 11.42 / 12.42,
-#: 1024^2 14.57 / 13.77, 1536^2 17.86 / 14.89); heat's band kernel outruns
-#: it at every size (64^2 2.98 / 1.09 .. 2048^2 1179 / 286).
-BAND_OVER_STANDARD_MIN_CELLS = 1 << 20
+#: cells from which the Euler band sweep outruns the standard kernel (us a
+#: step, band / standard: 384^2 18.6 / 18.5, 512^2 25.9 / 23.3, 576^2 28.2 /
+#: 31.0, 640^2 29.4 / 34.6, 768^2 36.8 / 43.8, 1024^2 56.6 / 67.6); heat's
+#: band kernel outruns it at every size (GCUPS, 64^2 2.98 / 1.09 .. 2048^2
+#: 1179 / 286).
+BAND_OVER_STANDARD_MIN_CELLS = 5 << 16
 
 
 def band_default(user_path, nv, ops, its, nx, ny):
@@ -280,6 +282,73 @@ def band_rows(spec, nx, ny, simds=BAND_SIMDS):
     m = -(-bands * -(-nx // rows) // simds)
     cost = numpy.where(m == 1, work / 0.815, m * work)
     return int(rows[len(cost) - 1 - int(numpy.argmin(cost[::-1]))])  # the longest of the cheapest
+
+
+#: wavefronts of a chain (band.inc's PS_BAND_CHAIN): one workgroup, one
+#: wavefront on each of a CU's SIMDs
+BAND_CHAIN = 4
+
+
+def has_band_chain(user_path):
+    """True when the plugin's band sweep works in chains (PS_HAS_BAND_CHAIN:
+    the wavefronts of a workgroup hand their segments' first rows to the
+    segment before)."""
+    return _defines_macro(user_path, "PS_HAS_BAND_CHAIN")
+
+
+def band_launch(spec, nx, ny, rows=None):
+    """(rows per wavefront, plan fields ``rows`` and ``chain``) of a
+    one-problem band launch over nx x ny: for a sweep that works in chains
+    the faster of chains and independent wavefronts (``band_chain_rows``),
+    else segments of ``band_rows``.  ``rows``: the segment asked for (a
+    chain of four takes four of it less the 2 rows its last wavefront gives
+    up for its work at the chain's end)."""
+    if spec.multi or not has_band_chain(spec.user_path):
+        rows = int(rows or band_rows(spec, nx, ny))
+        return rows, {"rows": rows, "chain": 0}
+    if rows is None:
+        rows, chain = band_chain_rows(spec, nx, ny)
+    else:
+        rows = int(rows)
+        rows, chain = (BAND_CHAIN * rows - 2, BAND_CHAIN) if rows >= 7 else (rows, 0)
+    return -(-(rows + 2) // BAND_CHAIN) if chain else rows, {"rows": rows, "chain": chain}
+
+
+def band_chain_rows(spec, nx, ny, simds=BAND_SIMDS):
+    """(rows, chain) of the fastest launch of a chaining band sweep over
+    nx x ny (Euler: two levels, radius 2), in units of one level's row of
+    one wavefront (about 1.0 us on MI355X).  A wavefront of n rows by itself
+    computes 2 n + 5 of them (four rows of level 1 beyond its own, two
+    faces); in a chain of four 2 n + 1, the last one 2 n + 5; its set-up
+    takes another.  The busiest SIMD runs m = ceil(wavefronts / SIMDs) of
+    them, two at a time (an odd last one by itself is slower), so of each
+    form only the shortest segments that keep m wavefronts are tried, for
+    each m; a launch adds about 4.5 units, a chain's barrier and one-level
+    steps another 0.8, and chains that fill the chip to the last workgroup
+    share CUs (640^2: 252 chains 31.2 us, 240 27.7).  Measured (us a step,
+    chosen / best of the other form): 384^2 3 rows each 18.2 / 24.1, 512^2 6
+    rows 24.2 / 24.9, 640^2 chains of 32 27.7 / 29.1, 1024^2 chains of 41
+    53.0 / 55.6, 1424 x 1128 65 76.5 / 83.6, 2048^2 158 177.1 / 176.8, 4096^2
+    152 rows each 691 / 691.  Against segments that recompute both ends
+    (band_rows): 1024^2 56.7, 2048^2 181.3."""
+    bands = -(-ny // band_out_columns(spec))
+    best = (float("inf"), min(nx, 128), 0)
+    for m in range(1, 33):
+        share = 1.12 if m == 1 else m + 0.6 * (m & 1)
+        segs = min(nx, m * simds // bands)
+        rows = -(-nx // segs) if segs else nx
+        if rows <= 256:
+            best = min(best, (1.04 * share * (2 * rows + 6) + 4.5, rows, 0))
+        if rows == 1:
+            break
+        segs = m * simds * 31 // 32 // BAND_CHAIN // bands
+        c = max(7 * BAND_CHAIN, -(-nx // segs) if segs else nx)
+        if c <= min(nx, 1024):
+            inner = -(-(c + 2) // BAND_CHAIN)
+            last = c - (BAND_CHAIN - 1) * ((c + 2) // BAND_CHAIN) - min(BAND_CHAIN - 1, (c + 2) % BAND_CHAIN)
+            work = max(2 * inner + 2, 2 * last + 6)
+            best = min(best, (1.02 * share * work + 5.3, c, BAND_CHAIN))
+    return best[1], best[2]
 
 
 def band_wave_work(spec):
