@@ -289,6 +289,9 @@ typedef struct ps_band_plan {
                        four wavefronts share `rows` rows and exchange their
                        segments' edges (a plugin sweep with
                        PS_HAS_BAND_CHAIN)                                  */
+    ps_function full; /* kernel of whole launches (BandFull: point-update
+                       plugins), or null: `band` takes every launch        */
+    int full_rows;  /* `full`: output rows per wavefront                   */
 } ps_band_plan;
 
 /* Run stages from absolute level A (which must be complete in the ring and

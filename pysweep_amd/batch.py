@@ -215,7 +215,8 @@ class PluginClass:
             spec = kernels.band_spec(self.cu, self.nv, self.ops, self.its, real=self.real)
             m = kernels.load(spec)
             self.modules.append(m)
-            self._band = (spec, m, m.get_function("Band"))
+            self._band = (spec, m, {"band": m.get_function("Band"),
+                                    "full": m.get_function("BandFull") if kernels.band_has_full(spec) else None})
         return self._band
 
     def band_multi(self):
@@ -967,7 +968,7 @@ class Engine:
                 if g0 < g1:
                     spec = band[0]
                     bplan = hip.BandPlan(state=t.ring.ptr, nx=t.nx, ny=t.ny, its=cls.its, T=T, levels=spec.levels,
-                                         wout=kernels.band_out_columns(spec), store_all=0, band=band[2],
+                                         wout=kernels.band_out_columns(spec), store_all=0, **band[2],
                                          **kernels.band_launch(spec, t.nx, t.ny)[1])
                     hip.band_run(bplan, cls.its - 2 + g0, g1 - g0)
                     self.band_stages += g1 - g0

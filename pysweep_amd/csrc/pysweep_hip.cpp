@@ -804,18 +804,16 @@ static int band_run(const ps_band_plan *p, int A, int stages)
     if (stages < 0) return fail("band solve: negative stage count");
     const int wout = p->wout;
     if (wout < 1 || wout > 128) return fail("band solve: output columns per band must be 1..128");
+    if (p->full && p->full_rows < 1) return fail("band solve: empty row segment of whole launches");
     if (p->chain != 0 && p->chain != 4) return fail("band solve: a chain has 4 wavefronts (0: no chains)");
     ps_band_grid g;
     g.nx = p->nx;
     g.ny = p->ny;
     g.T = p->T;
-    g.rows = p->rows;
     g.bands = (p->ny + wout - 1) / wout;
-    g.segs = (p->nx + p->rows - 1) / p->rows;
-    g.chain = p->chain;
-    const long long parts = static_cast<long long>(g.bands) * g.segs;  // wavefronts, or chains
-    if (parts > (1LL << 30)) return fail("band solve: grid too large");
-    const unsigned groups = static_cast<unsigned>(g.chain ? parts : (parts + 3) / 4);
+    const int least = p->full && p->full_rows < p->rows ? p->full_rows : p->rows;
+    if (static_cast<long long>(g.bands) * ((p->nx + least - 1) / least) > (1LL << 30))
+        return fail("band solve: grid too large");
     void *state = p->state;
     for (int done = 0; done < stages;) {
         g.hh = stages - done < H ? stages - done : H;
@@ -823,9 +821,15 @@ static int band_run(const ps_band_plan *p, int A, int stages)
         // last launch leaves its last s levels complete
         const bool last = done + g.hh >= stages;
         g.wlo = p->store_all ? 1 : !last ? g.hh : (g.hh - s + 1 > 1 ? g.hh - s + 1 : 1);
+        const bool full = p->full && g.hh == H && g.wlo == H;
+        g.rows = full ? p->full_rows : p->rows;
+        g.chain = full ? 0 : p->chain;
+        g.segs = (p->nx + g.rows - 1) / g.rows;
+        const long long parts = static_cast<long long>(g.bands) * g.segs;  // wavefronts, or chains
+        const unsigned groups = static_cast<unsigned>(g.chain ? parts : (parts + 3) / 4);
         int gts = A - (s - 1) + 1;
         void *args[] = {&state, &gts, &A, &g};
-        if (int rc = launch_kind(p->band, groups, 256, args, PS_K_BAND)) return rc;
+        if (int rc = launch_kind(full ? p->full : p->band, groups, 256, args, PS_K_BAND)) return rc;
         A += g.hh;
         done += g.hh;
     }

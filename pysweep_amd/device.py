@@ -250,6 +250,8 @@ class BandRun(_Run):
         self.plan = hip.BandPlan(state=self.ring.ptr, nx=nx, ny=ny, its=its, T=self.T, levels=self.spec.levels,
                                  wout=kernels.band_out_columns(self.spec), store_all=0,
                                  band=mod.get_function("Band"), **shape)
+        if self.plan.full_rows:
+            self.plan.full = mod.get_function("BandFull")
 
     def run(self, times, on_level=None, stats=None):
         """The ``times.stages + times.tail`` stages of a swept schedule

@@ -19,14 +19,19 @@ __device__ __constant__ double ALPHA;
 __device__ __constant__ double COURANT;
 __device__ __constant__ int SCHEME; /* 1: forward Euler, 0: RK2 */
 
+/* COURANT*(p - 2c + m).  2c is exact, so p - 2c is one fused operation with
+ * the same rounding. */
+__device__ __forceinline__ double heat_second(double p, double c, double m)
+{
+    return COURANT * (__builtin_fma(-2.0, c, p) + m);
+}
+
 /* arithmetic in double; R is the storage type of the state */
 template <class R>
 __device__ __forceinline__ double heat_laplace(const R *u, int idx)
 {
     const double c = u[idx];
-    const double lx = COURANT * ((double)u[idx + SY] - 2 * c + (double)u[idx - SY]);
-    const double ly = COURANT * ((double)u[idx + 1] - 2 * c + (double)u[idx - 1]);
-    return lx + ly;
+    return heat_second(u[idx + SY], c, u[idx - SY]) + heat_second(u[idx + 1], c, u[idx - 1]);
 }
 
 /*
@@ -67,13 +72,15 @@ template <>
 __device__ __forceinline__ float heat_store<float>(double x, int globalTimeStep)
 {
     const unsigned long long b = (unsigned long long)__double_as_longlong(x);
-    const int e = (int)((b >> 52) & 0x7ff);
-    if (e < 1023 - 126 || e >= 1023 + 127)
-        return (float)x;
     constexpr unsigned long long low = (1ULL << 29) - 1;
     const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+    /* exponent field in [1023 - 126, 1023 + 127): one subtraction without the
+     * sign, and a choice, not a branch, which would keep the compiler from
+     * interleaving a sweep's levels */
+    const bool normal = (hi << 1) - ((1023U - 126) << 21) < (253U << 21);
     const unsigned r = heat_mix(lo ^ __builtin_rotateleft32(hi, 13) ^ (0x9e3779b9U * (unsigned)(globalTimeStep + 1)));
-    return (float)__longlong_as_double((long long)((b + (r & low)) & ~low));
+    const unsigned long long up = (b + (r & low)) & ~low;
+    return (float)__longlong_as_double((long long)(normal ? up : b));
 }
 
 template <class R>
@@ -111,12 +118,12 @@ template <class R, int V>
 __device__ __forceinline__ R ps_point(double c, double xm, double xp, double ym, double yp, double prev,
                                       int globalTimeStep)
 {
-    const double lx = COURANT * (xp - 2 * c + xm);
-    const double ly = COURANT * (yp - 2 * c + ym);
-    const double d = lx + ly;
+    const double d = heat_second(xp, c, xm) + heat_second(yp, c, ym);
     if (V == 1) return heat_store<R>(d + c, globalTimeStep);
-    if (globalTimeStep % 2 == 0) return heat_store<R>(1.0 * d + prev, globalTimeStep);
-    return heat_store<R>(0.5 * d + c, globalTimeStep);
+    /* one expression for both stages (1.0 * d is d): where the stage's parity
+     * is known only at run time, two would be evaluated side by side */
+    const bool fin = globalTimeStep % 2 == 0;
+    return heat_store<R>((fin ? 1.0 : 0.5) * d + (fin ? prev : c), globalTimeStep);
 }
 
 /*

@@ -48,7 +48,7 @@ class StandardPlan(ctypes.Structure):
 class BandPlan(ctypes.Structure):
     _fields_ = [("state", c_void_p), ("nx", c_int), ("ny", c_int), ("its", c_int), ("T", c_int),
                 ("levels", c_int), ("wout", c_int), ("rows", c_int), ("store_all", c_int), ("band", c_void_p),
-                ("chain", c_int)]
+                ("chain", c_int), ("full", c_void_p), ("full_rows", c_int)]
 
 
 class Inst(ctypes.Structure):

@@ -296,6 +296,43 @@ def has_band_chain(user_path):
     return _defines_macro(user_path, "PS_HAS_BAND_CHAIN")
 
 
+def band_has_full(spec):
+    """Whether a band module has a kernel of its own for whole launches
+    (BandFull: the point-update plugins)."""
+    return spec.kind == "band" and not spec.multi and has_point_update(spec.user_path)
+
+
+def band_full_rows(spec, nx, ny, simds=BAND_SIMDS):
+    """Output rows per wavefront of a whole launch (BandFull): the segment
+    minimising the busiest SIMD's time.  It runs m = ceil(wavefronts / SIMDs)
+    wavefronts, each the launch's start, worth about 14 rows of the steady
+    state, and its rows, in groups of three (the loop's step); a wavefront
+    alone on its SIMD issues about 16 % slower than two, and with a 32-bit
+    state, whose registers leave room for a third and whose rounding waits on
+    multiplications, 20 %, two 3 %.  Of each m only the shortest segments are
+    tried.  Measured on MI355X (heat, 12 levels, us a
+    launch, * the choice): 64^2 rows 3* 10.6, 6 12.1, 16 18.3; 384^2 3* 11.6,
+    6 13.0, 12 16.3; 1024^2 12* 18.1, 6 22.0, 24 24.0; 2048^2 42* 36.8, 24
+    40.8, 64 48.5; 4096^2 81* 101.6, 42 113.3, 164 112.8; 8192^2 about 328*
+    367.5, 216 374.5, 128 376.2, 64 416.6; 32-bit state, 8 levels: 1024^2
+    12* 22.4, 24 33.3; 4096^2 75* 143.1, 24 172.6, 152 161.3; 8192^2 about
+    200* 511.4, 306 531.3, 100 512.9."""
+    alone = {1: 1.2, 2: 1.03} if spec.real == "float" else {1: 1.16}
+    bands = -(-ny // band_out_columns(spec))
+    best = None
+    for m in range(1, 65):
+        segs = min(nx, m * simds // bands)
+        if not segs:
+            continue
+        rows = 3 * -(-nx // (3 * segs))
+        cost = m * (14 + rows) * alone.get(m, 1.0)
+        if best is None or cost < best[0]:
+            best = (cost, rows)
+        if rows == 3:
+            break
+    return best[1] if best else nx
+
+
 def band_launch(spec, nx, ny, rows=None):
     """(rows per wavefront, plan fields ``rows`` and ``chain``) of a
     one-problem band launch over nx x ny: for a sweep that works in chains
@@ -303,6 +340,9 @@ def band_launch(spec, nx, ny, rows=None):
     else segments of ``band_rows``.  ``rows``: the segment asked for (a
     chain of four takes four of it less the 2 rows its last wavefront gives
     up for its work at the chain's end)."""
+    if band_has_full(spec):
+        full = int(rows or band_full_rows(spec, nx, ny))
+        return full, {"rows": int(rows or band_rows(spec, nx, ny)), "chain": 0, "full_rows": full}
     if spec.multi or not has_band_chain(spec.user_path):
         rows = int(rows or band_rows(spec, nx, ny))
         return rows, {"rows": rows, "chain": 0}
