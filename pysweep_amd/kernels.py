@@ -546,19 +546,28 @@ def level_scratch_bytes(user_path, generic, sx, sy, faces, kind="swept"):
     return 0 if f is None else 8 * f(sx * sy, faces)
 
 
-def default_slots(nv, its, b, P, real_bytes=8, scratch=0, least=None):
-    """LDS window for a swept tile: the largest within ~28 KB including the
-    level scratch, at least ``least`` (default ITS+1) levels.  Smaller
-    windows slide more often but let more tiles share a CU, which hides the
-    HBM latency of each level's face loads.  Measured on MI355X: Euler
-    1024^2 b=16 with the level update (12 KB scratch) 3 levels 4.7 GCUPS,
-    4 levels 3.9, and in a later build 2 levels in place 6.5 against 3
-    levels 6.0; heat 8192^2 b=32 2 levels 175, 3 levels 180, 5 levels 163;
-    b=64 2 levels 245."""
-    level = nv * b * b * real_bytes
+def default_slots(nv, its, b, P, real_bytes=8, scratch=0, least=None, level_update=False, pad=0):
+    """LDS window (levels) of a swept tile.
+
+    A level update takes the fewest it can run in: more levels keep nothing
+    that it reads, and cost workgroups per CU.  Measured on MI355X, 300 steps
+    of heat 1024^2: b=16 2 levels 2155 us, 13 2691; b=8 2 levels 3373, 7 4316;
+    b=16 RK2 2 levels 4582, 13 8915; b=32 2 or 3 levels 1170; Euler 2048^2
+    b=16 with FP32 state 2 levels 11.9 GCUPS, 4 levels 11.0.
+
+    The per-cell step takes 2 ITS + 1, from where on its window turns over
+    without a copy of its own, if two such tiles fit a CU (heat 4096^2 b=64:
+    one workgroup of 3 levels 7563 us, two of 2 levels 5998; and a plugin's
+    own LDS still has room), else the fewest.  Heat 1024^2: b=32 3 levels
+    1177 us, 2 levels 1429; RK2 5 levels 2515, 3 levels 3355; b=16 3 levels
+    2212, 14 3028; Euler 1024^2 b=16 5 levels 16.6 ms, 3 levels 17.4."""
+    level = nv * b * (b + pad) * real_bytes
     full = 2 * P + its
     least = its + 1 if least is None else least
-    return max(least, min(full, (28 * 1024 - scratch) // level))
+    if level_update:
+        return least
+    long = min(full, 2 * its + 1)
+    return long if long > least and 2 * (long * level + scratch) <= LDS_MAX else least
 
 
 def default_pfd(nv, b, threads, real_bytes):
@@ -611,16 +620,8 @@ def swept_spec(user_path, nv, ops, its, b, slots=None, threads=None, lds_budget=
     scratch = level_scratch_bytes(user_path, generic, b, b + pad, swept_faces(b, ops))
     least = min_slots(user_path, its, generic)
     if slots is None:
-        sc = None if generic else level_scratch(user_path)
-        if sc is not None and sc(0, 1) > sc(0, 0) and level_in_place(user_path, generic):
-            # a level update that shares faces through LDS is bound by VALU
-            # issue, not by the face loads a longer window would hide, and
-            # each level it keeps costs a workgroup's LDS: the fewest levels
-            # (Euler 2048^2 b=16 with FP32 state: 2 levels 11.9 GCUPS, 4
-            # levels 11.0)
-            slots = least
-        else:
-            slots = default_slots(nv, its, b, P, rb, scratch, least)
+        slots = default_slots(nv, its, b, P, rb, scratch, least,
+                              not generic and has_level_update(user_path), pad)
     slots = min(slots, full)
     if slots < least:
         raise ValueError(f"an LDS window needs at least {least} levels here "
