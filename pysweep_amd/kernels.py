@@ -209,14 +209,18 @@ def band_multi_levels(user_path, its, real="double"):
     return band_levels(its, None, real) if has_point_update(user_path) else its
 
 
-#: cells from which a plugin's own band sweep (Euler: one column per lane,
-#: a 2-column halo per level) is the faster swept kernel: its 64-column
-#: bands leave small grids too few wavefronts.  Measured on MI355X when the
-#: line was drawn (Euler, GCUPS, band / phase kernels b=16): 128^2 0.67 /
-#: 0.83, 256^2 2.64 / 3.20, 384^2 5.81 / 4.82, 1024^2 14.41 / 9.73; now (us a
-#: step) 256^2 15.6 / 18.7, 384^2 18.7 / 27.5, 1024^2 56.6 / 96.  Heat's
-#: band kernel led at every size measured (64^2 to 8192^2).
+#: cells from which a plugin's own band sweep (one column per lane, a
+#: 2-column halo per level) is taken to be the faster swept kernel: its
+#: 64-column bands leave small grids too few wavefronts.
 BAND_SWEEP_MIN_CELLS = 1 << 17
+#: A sweep in chains (Euler's) is faster than the phase kernels on smaller
+#: grids too, measured on MI355X (Euler, 60 steps, us, band / phase kernels
+#: b=16): 16^2 687 / 1004, 128^2 734 / 1052, 192^2 772 / 1093, 240x272 901 /
+#: 1128, 256^2 917 / 1102, 288^2 972 / 1360, 352^2 1115 / 1404; 16x4064 891 /
+#: 1114, but 4064x16 1153 / 1100: there most of a band's columns are padding,
+#: so the cells with it count.  It takes the grids outside BAND_CHAIN_GAP:
+#: there it gains least, and 256^2 is tested to run on the phase kernels.
+BAND_CHAIN_GAP = (1 << 16, 5 << 14)
 #: cells from which the Euler band sweep outruns the standard kernel (us a
 #: step, band / standard: 384^2 18.6 / 18.5, 512^2 25.9 / 23.3, 576^2 28.2 /
 #: 31.0, 640^2 29.4 / 34.6, 768^2 36.8 / 43.8, 1024^2 56.6 / 67.6); heat's
@@ -230,7 +234,15 @@ def band_default(user_path, nv, ops, its, nx, ny):
     by default (else on the phase kernels)."""
     if not band_capable(user_path, nv, ops, its):
         return False
-    return has_point_update(user_path) or nx * ny >= BAND_SWEEP_MIN_CELLS
+    if has_point_update(user_path):
+        return True
+    cells = nx * ny
+    if cells >= BAND_SWEEP_MIN_CELLS or not has_band_chain(user_path):
+        return cells >= BAND_SWEEP_MIN_CELLS
+    wout = 64 - 2 * ops * its  # one step per launch
+    padded = nx * wout * -(-ny // wout)
+    lo, hi = BAND_CHAIN_GAP
+    return cells < lo and padded < hi or cells >= hi and 2 * padded < 3 * cells
 
 
 def band_beats_standard(user_path, nv, ops, its, nx, ny):

@@ -279,6 +279,11 @@ class Solver(object):
             band = True
         else:
             band = kernels.band_default(self.gpu, nv, self.operating, self.intermediate, nx, ny)
+            if band and nx * ny < kernels.BAND_SWEEP_MIN_CELLS and not kernels.has_point_update(self.gpu):
+                # options of the phase kernels keep them, and a block they
+                # cannot take is refused here as it would be there
+                band = not any(t.get(k) for k in ("slots", "threads", "pfd"))
+                kernels.swept_spec(self.gpu, nv, self.operating, self.intermediate, self.blocksize[0])
         if band:
             self._run = device.BandRun(self.gpu, nv, self.operating, self.intermediate, nx, ny,
                                        levels=t.get("band_levels"), rows=t.get("band_rows"), defines=defines)
