@@ -340,6 +340,10 @@ typedef struct ps_multi_plan {
     void *bowner;       /* device int[total_bwaves]                         */
     int total_bwaves;   /* band work items: one wavefront (a workgroup) each */
     ps_function band;   /* BandMulti of the class's band module, or null    */
+    int band_step;      /* levels of a BandMulti launch if every active     */
+                        /* band-method problem begins one at each run's     */
+                        /* first round ((c - 1) a multiple of it): launched */
+                        /* on each band_step-th round only; 0: on every one */
 } ps_multi_plan;
 
 /* Fill the owner tables of a plan from its prefix sums on the work stream
@@ -347,8 +351,10 @@ typedef struct ps_multi_plan {
 int ps_multi_index(const ps_multi_plan *plan);
 
 /* Run `rounds` rounds: each round launches UpPyramidMulti, XBridgeMulti,
- * OctahedronMulti, DownPyramidMulti, YBridgeMulti, StandardMulti, BandMulti
- * and ps_advance; every problem executes the phases of its own cycle c (a
+ * OctahedronMulti, DownPyramidMulti, YBridgeMulti, StandardMulti and
+ * BandMulti (with band_step: the rounds that begin a launch only, and rounds
+ * is a multiple of it), the run ends with one ps_advance; every problem
+ * executes the phases of its own cycle c (a
  * band-method problem one whole step on the rounds whose stage begins one,
  * nothing on the others). */
 int ps_multi_run(const ps_multi_plan *plan, int rounds);

@@ -547,12 +547,12 @@ class _ClassTable:
         """True when the table's run flags differ from ``active``."""
         return self.flags != tuple(t in active for t in self.running)
 
-    def rebuild(self, active=None, stage=None):
+    def rebuild(self, active=None, stage=None, graph_rounds=0):
         """Write the table of the running problems (those in ``active``, or
         all, take part in the rounds).  ``stage(nbytes)`` returns a page-locked
         buffer that stays untouched until the copies queued now have run; the
         table goes to the device from it without waiting.  Without it the
-        copies wait."""
+        copies wait.  ``graph_rounds``: rounds of a captured graph, 0 if none."""
         cls = self.cls
         n = len(self.running)
         if n == 0:
@@ -639,10 +639,23 @@ class _ClassTable:
                                   advance=f["advance"],
                                   bprefix=self.bprefix.ptr,
                                   bowner=self.bowner.ptr if getattr(self, "bowner", None) else None,
-                                  total_bwaves=int(bpre[-1]), band=f.get("BandMulti"))
+                                  total_bwaves=int(bpre[-1]), band=f.get("BandMulti"),
+                                  band_step=self._band_step(banded, graph_rounds))
         hip.multi_index(self.plan)
         self.graph = None
         self.dirty = False
+
+    def _band_step(self, banded, graph_rounds):
+        """Rounds between BandMulti launches: a host step's rounds are whole
+        launches of every band-method problem (``Engine._band_rounds``), so
+        all of a class begin theirs on the same rounds, and on the others (1
+        of 2 for Euler, 11 of 12 for heat) each work item would leave at once.
+        0, a launch on every round, where they do not or where a captured
+        graph is no whole number of launches."""
+        h = self.cls.band_h
+        if not banded or any((t.c - 1) % h for t in banded) or graph_rounds % h:
+            return 0
+        return h
 
 
 def short_first(running, now, capacity=1 << 20, max_wait=2.0):
@@ -1026,7 +1039,7 @@ class Engine:
         R = self._band_rounds(active, self._rounds_ahead(active))
         for key, tab in self.tables.items():
             if tab.dirty or tab.needs(active):
-                tab.rebuild(active, stage=self._stage)
+                tab.rebuild(active, self._stage, self.graph_rounds if self.use_graphs else 0)
             if tab.plan is None or not any(tab.flags):
                 continue
             K = self.graph_rounds

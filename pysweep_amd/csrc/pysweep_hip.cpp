@@ -873,12 +873,12 @@ __global__ void ps_owner_kernel(const int *__restrict__ prefix, int n, int *__re
     for (int t = lo + threadIdx.x; t < hi; t += blockDim.x) owner[t] = i;
 }
 
-static int multi_round(const ps_multi_plan *p)
+// Round `ahead` of a run: the table holds the counters of its first.
+static int multi_round(const ps_multi_plan *p, int ahead)
 {
     void *insts = p->insts, *prefix = p->prefix, *sprefix = p->sprefix, *owner = p->owner, *sowner = p->sowner;
-    int n = p->ninst;
-    void *args[] = {&insts, &prefix, &owner, &n};
-    void *sargs[] = {&insts, &sprefix, &sowner, &n};
+    void *args[] = {&insts, &prefix, &owner, &ahead};
+    void *sargs[] = {&insts, &sprefix, &sowner, &ahead};
     int rc = 0;
     if (p->total_tiles > 0) {
         const unsigned g = static_cast<unsigned>(p->total_tiles);  // one workgroup per work item
@@ -895,14 +895,13 @@ static int multi_round(const ps_multi_plan *p)
         const unsigned g = static_cast<unsigned>(p->total_stiles);
         if ((rc = launch_kind(p->standard, g, static_cast<unsigned>(p->sthreads), sargs, PS_K_STANDARD))) return rc;
     }
-    if (p->total_bwaves > 0 && p->band) {
+    if (p->total_bwaves > 0 && p->band && (p->band_step < 2 || ahead % p->band_step == 0)) {
         void *bprefix = p->bprefix, *bowner = p->bowner;
-        void *bargs[] = {&insts, &bprefix, &bowner, &n};
+        void *bargs[] = {&insts, &bprefix, &bowner, &ahead};
         // one wavefront per workgroup: the workgroup's LDS holds its problem's constants
         if ((rc = launch_kind(p->band, static_cast<unsigned>(p->total_bwaves), 64, bargs, PS_K_BAND))) return rc;
     }
-    void *aargs[] = {&insts, &n};
-    return launch(p->advance, static_cast<unsigned>((n + 255) / 256), 256, aargs);
+    return 0;
 }
 
 int ps_level_sums(const void *level, int fp32, int nv, size_t cells, double *sums)
@@ -960,11 +959,18 @@ int ps_multi_run(const ps_multi_plan *plan, int rounds)
         return fail("multi plan with band work items but no BandMulti kernel");
     if (plan->total_tiles > 0 && (!plan->up || !plan->ybridge || !plan->xbridge || !plan->octahedron || !plan->down))
         return fail("multi plan without phase kernels");
+    if (plan->band_step < 0) return fail("multi plan: negative band_step");
+    if (plan->total_bwaves > 0 && plan->band_step > 1 && rounds % plan->band_step)
+        return fail("multi plan: with band_step a run takes a multiple of it");
     for (int r = 0; r < rounds; ++r) {
-        int rc = multi_round(plan);
+        int rc = multi_round(plan, r);
         if (rc) return rc;
     }
-    return 0;
+    if (rounds <= 0) return 0;
+    void *insts = plan->insts;
+    int n = plan->ninst;
+    void *args[] = {&insts, &n, &rounds};
+    return launch(plan->advance, static_cast<unsigned>((n + 255) / 256), 256, args);
 }
 
 int ps_multi_run_timed(const ps_multi_plan *plan, int rounds, ps_run_stats *stats)

@@ -66,7 +66,8 @@ class MultiPlan(ctypes.Structure):
                 ("threads", c_int), ("sthreads", c_int),
                 ("up", c_void_p), ("ybridge", c_void_p), ("xbridge", c_void_p), ("octahedron", c_void_p),
                 ("down", c_void_p), ("standard", c_void_p), ("advance", c_void_p),
-                ("bprefix", c_void_p), ("bowner", c_void_p), ("total_bwaves", c_int), ("band", c_void_p)]
+                ("bprefix", c_void_p), ("bowner", c_void_p), ("total_bwaves", c_int), ("band", c_void_p),
+                ("band_step", c_int)]
 
 
 class RunStats(ctypes.Structure):
