@@ -134,10 +134,11 @@ def solo_swept_spec(plugin, precision, its, b):
 def solo_specs(plugin, precision, its, b):
     """The plain modules a class uses for a problem running alone: the
     swept phases and the standard modules of the tiles its grids can take
-    (a tile no larger than the grid; the tile depends on the grid only
-    through that bound)."""
+    (a tile no larger than the grid; else the tile depends on the grid only
+    through the rounds of its workgroups: 256 x 256 has the other tile of
+    a shared-face update, see ``kernels.standard_spec``)."""
     out = [solo_swept_spec(plugin, precision, its, b)]
-    sides = [s for s in (16, 32, 64, 128, 1 << 16) if s >= b]
+    sides = [s for s in (16, 32, 64, 128, 256, 1 << 16) if s >= b]
     for nx in sides:
         for ny in sides:
             spec = solo_standard_spec(plugin, precision, its, nx, ny)

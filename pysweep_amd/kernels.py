@@ -657,6 +657,25 @@ def swept_spec(user_path, nv, ops, its, b, slots=None, threads=None, lds_budget=
                       unroll=int(unroll))
 
 
+#: compute units of the device
+CUS = 256
+
+
+def _fewer_rows(nx, ny):
+    """Whether a 15 x 16 tile beats a 16 x 16 one for a problem of its own,
+    for a level update that shares faces.  The lanes work in wavefronts: 16 x 16 cells
+    have 272 faces a direction, five wavefronts the last of which has 16
+    lanes, 15 x 16 have 256 and 255, four full ones.  Measured on MI355X
+    (Euler, us a step, 15 x 16 / 16 x 16): 128^2 9.8 / 11.3, 384^2 15.4 /
+    18.0, 1000x1500 94.3 / 105.5, 1536^2 146 / 160, 2048^2 258 / 295, with
+    32-bit state 246 / 274; but 256^2 12.5 / 11.7 and 352^2 15.1 / 15.0, where
+    the smaller tiles take another round of the CUs.  With R rounds these are
+    7.1 + 2.75 R and 8.3 + 3.3 R up to five rounds, and beyond the ratio of
+    the slopes decides."""
+    rounds = lambda bx: -(-(-(-nx // bx) * -(-ny // 16)) // CUS)  # noqa: E731
+    return 7.1 + 2.75 * rounds(15) < 8.3 + 3.3 * rounds(16)
+
+
 def standard_tile(nv, ops, its, nx, ny, lds_budget=LDS_BUDGET, real_bytes=8, scratch=None, threads=256,
                   slots=None):
     """Tile (bx rows, by columns) for the standard kernel: most cells within
@@ -712,6 +731,9 @@ def standard_spec(user_path, nv, ops, its, nx, ny, bx=None, by=None, threads=Non
     if bx is None or by is None:
         bx, by = standard_tile(nv, ops, its, nx, ny, lds_budget, 8 if real == "double" else 4, sc, threads,
                                standard_slots(user_path, its, generic))
+        # (a batch keeps 16 rows: its short problems would end in tiles of a row or two)
+        if (bx, by) == (16, 16) and not multi and sc is not None and sc(0, 1) > sc(0, 0) and _fewer_rows(nx, ny):
+            bx = 15
     if bx > nx or by > ny:
         raise ValueError("standard tile larger than the grid")
     return ModuleSpec("standard", os.path.abspath(user_path), nv, ops, its, bx=bx, by=by, threads=threads,
@@ -767,12 +789,13 @@ def shipped_module_specs():
     specs.append(swept_spec(hf, 1, 1, 2, 8))
     for (path, nv, k, s) in ((heat, 1, 1, 1), (heat, 1, 1, 2), (euler, 4, 2, 2), (ex, 1, 1, 1), (ex, 1, 2, 2),
                              (ch, 1, 1, 1), (ch, 1, 2, 2), (hf, 1, 1, 2)):
-        for n in (64, 384, 1024):
+        for n in (64, 256, 384, 1024):  # (Euler: both tiles of its rule)
             specs.append(standard_spec(path, nv, k, s, n, n))
     # the Euler modules with IEEE division (a solve repeated after a state
     # left the fast division's range)
     specs.append(swept_spec(euler, 4, 2, 2, 16, defines=("EU_EXACT_DIVISION",)))
-    specs.append(standard_spec(euler, 4, 2, 2, 64, 64, defines=("EU_EXACT_DIVISION",)))
+    for n in (64, 256):
+        specs.append(standard_spec(euler, 4, 2, 2, n, n, defines=("EU_EXACT_DIVISION",)))
     for s_ in (1, 2):
         specs.append(band_spec(heat, 1, 1, s_))
     specs.append(band_spec(eq_path("heat_fp32.cu"), 1, 1, 1, real="float"))
@@ -780,7 +803,8 @@ def shipped_module_specs():
     specs.append(band_spec(euler, 4, 2, 2, defines=("EU_EXACT_DIVISION",)))
     specs.append(band_spec(eq_path("euler_fp32.cu"), 4, 2, 2, real="float"))
     for name, nv, k, s in (("euler_fp32.cu", 4, 2, 2), ("heat_fp32.cu", 1, 1, 1)):
-        specs.append(standard_spec(eq_path(name), nv, k, s, 1024, 1024, real="float"))
+        for n in (256, 1024):
+            specs.append(standard_spec(eq_path(name), nv, k, s, n, n, real="float"))
         for b in ((16, 32) if nv > 1 else (16, 32, 64)):
             specs.append(swept_spec(eq_path(name), nv, k, s, b, real="float"))
     seen, out = set(), []
