@@ -222,11 +222,12 @@ BAND_SWEEP_MIN_CELLS = 1 << 17
 #: there it gains least, and 256^2 is tested to run on the phase kernels.
 BAND_CHAIN_GAP = (1 << 16, 5 << 14)
 #: cells from which the Euler band sweep outruns the standard kernel (us a
-#: step, band / standard: 384^2 18.6 / 18.5, 512^2 25.9 / 23.3, 576^2 28.2 /
-#: 31.0, 640^2 29.4 / 34.6, 768^2 36.8 / 43.8, 1024^2 56.6 / 67.6); heat's
-#: band kernel outruns it at every size (GCUPS, 64^2 2.98 / 1.09 .. 2048^2
-#: 1179 / 286).
-BAND_OVER_STANDARD_MIN_CELLS = 5 << 16
+#: step, band / standard with its 15-row tiles: 384^2 18.2 / 15.5, 512^2 24.5
+#: / 21.9, 608^2 30.7 / 27.8, 640^2 28.2 / 28.4, 704^2 32.6 / 34.0, 512x1024
+#: 32.6 / 35.3, 1024x512 35.1 / 35.1, 1024^2 56.6 / 62.7; 32-bit state crosses
+#: at the same size); heat's band kernel outruns it at every size (GCUPS, 64^2
+#: 2.98 / 1.09 .. 2048^2 1179 / 286).
+BAND_OVER_STANDARD_MIN_CELLS = 25 << 14
 
 
 def band_default(user_path, nv, ops, its, nx, ny):
