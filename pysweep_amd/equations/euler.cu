@@ -94,47 +94,62 @@ __device__ __forceinline__ eu_q eu_at(const S &s, int i)
 }
 
 /*
- * Division.  n/d is formed as the gfx950 compiler's IEEE double division
- * forms it -- reciprocal estimate, refinement, product, one residual
- * correction, special-case fix-up -- less its operand-scaling steps, which
- * leave every value unchanged unless an operand lies within 2^53 of the
- * subnormal range, d is subnormal or the exponents differ by 768 or more (no
- * Euler state comes near).  The estimate's relative error e (about 2^-23 at
- * most) is removed to third order, y + y*(e + e*e), in three instructions
- * (two Newton steps take four): the reciprocal is 1/d to within 2^-68 before
- * its final rounding, and the residual correction makes the quotient the
- * correctly rounded one, bitwise the one `n / d` gives.  The refined
- * reciprocal depends on d alone, so the quotients that share a denominator
- * share it.
+ * Division.  n/d is formed as a correctly rounded double division without
+ * operand scaling: reciprocal estimate, refinement, product, one residual
+ * correction, special-case fix-up.  (Scaling changes nothing unless an operand
+ * lies within 2^53 of the subnormal range, d is subnormal or the exponents
+ * differ by 768 or more: no Euler state comes near.)  The refined reciprocal
+ * depends on d alone, so the quotients that share a denominator share it.
+ *
+ * How good the reciprocal y has to be: the corrected quotient is the
+ * correctly rounded one unless y is the wrong neighbour of 1/d (the farther
+ * number) and d = 2^j (1 - k 2^-53) with k 2^-53 at most about 1/d's distance
+ * to the midpoint of its neighbours, in units of their distance.  For small
+ * odd k the reciprocals lie k^2 2^-54 above a midpoint and have to be rounded
+ * up; a uniform stream's densities are such numbers.  eu_recip_from sees to it
+ * whatever the estimates.  Of what is cheaper, one third-order step from the
+ * hardware's estimate, y + y*(e + e*e), left some quotients one ulp off for k
+ * around 2^27 sqrt(m), two Newton steps for k = 5 (the numerators hardest to
+ * round, found on MI355X).  Against the third-order step the two instructions
+ * more cost 1.8 % (Euler 1024^2 53.1 -> 54.1 us a step, standard kernel
+ * 1000 x 1500 83.6 -> 85.1).
  */
 struct eu_rcp {
     double d, y; /* denominator, refined reciprocal */
 };
 
-__device__ __forceinline__ eu_rcp eu_recip(double d)
-{
-    const double y = __builtin_amdgcn_rcp(d);
-    const double e = __builtin_fma(-d, y, 1.0);
-    eu_rcp q;
-    q.d = d;
-    q.y = __builtin_fma(y, __builtin_fma(e, e, e), y);
-    return q;
-}
-
-/* The reciprocal of d from an estimate y of it, good to 2^-45.  One Newton
- * step leaves 1/d less up to 2^-90; the 2^-88 added to the residual puts the
- * value above 1/d instead.  That matters for a significand of all ones,
- * d = 2^k (1 - 2^-53), as the densities of a uniform stream are: its
- * reciprocal lies 2^-106 above the midpoint of two numbers, and rounded
- * down it would make 2^j/d one ulp too small (the reciprocal instruction
- * returns the upper number there for the same reason).  Of every other d
- * either neighbour gives the correctly rounded quotients. */
+/* The reciprocal of d from an estimate y of it good to 2^-44.3.  One Newton
+ * step leaves 1/d less up to 2^-88.6; the 2^-88 added to the residual puts
+ * the value above 1/d instead.  A value 2^-88 too large is the wrong
+ * neighbour only of reciprocals less than 2^-36 below a midpoint, and of
+ * those there are none with k < 2^17, so no quotient is wrong. */
 __device__ __forceinline__ eu_rcp eu_recip_from(double d, double y)
 {
     eu_rcp q;
     q.d = d;
     q.y = __builtin_fma(y, __builtin_fma(-d, y, 1.0) + 0x1p-88, y);
     return q;
+}
+
+/* The hardware's estimate is good to e = 2^-23, a Newton step makes it e^2. */
+__device__ __forceinline__ eu_rcp eu_recip(double d)
+{
+    const double y = __builtin_amdgcn_rcp(d);
+    return eu_recip_from(d, __builtin_fma(y, __builtin_fma(-d, y, 1.0), y));
+}
+
+/* 1/d, correctly rounded.  The third-order step leaves a neighbour of 1/d and
+ * the residual correction 1/d less 2^-106 at most, on the right side of every
+ * midpoint but that of k = 1, where the reciprocal instruction returns the
+ * upper neighbour itself (tested at every exponent). */
+__device__ __forceinline__ double eu_inverse(double d)
+{
+    if (EU_EXACT)
+        return 1.0 / d;
+    double y = __builtin_amdgcn_rcp(d);
+    const double e = __builtin_fma(-d, y, 1.0);
+    y = __builtin_fma(y, __builtin_fma(e, e, e), y);
+    return __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
 }
 
 /* the reciprocal of 2d from that of d: doubling d halves every step of
@@ -188,10 +203,12 @@ __device__ __forceinline__ double eu_sqrt(double x)
     return (x == 0.0 || x == __builtin_inf()) ? x : g;
 }
 
-/* sqrt(x) and the reciprocals of x and (to about 2^-44) of sqrt(x), for a
- * density x in the range above.  The square root is eu_sqrt's without its
- * special cases; its refinement also gives 1/sqrt(x), whose square is the
- * estimate of 1/x, so a density costs one transcendental instruction (a
+/* sqrt(x) and the reciprocals of x and (an estimate) of sqrt(x), for a density
+ * x in the range above.  The square root is eu_sqrt's without its
+ * special cases; its refinement also gives 1/sqrt(x), off by 1.5 e^2 for a
+ * hardware estimate good to e <= 2^-23.  Its square is the estimate of 1/x and
+ * the product of two that of a Roe density's reciprocal (3 e^2 = 2^-44.4, as
+ * eu_recip_from wants it), so a density costs one transcendental instruction (a
  * quarter of the issue rate) instead of two. */
 struct eu_root {
     double s, y; /* sqrt(x), estimate of 1/sqrt(x) */
@@ -295,11 +312,11 @@ __device__ __forceinline__ eu_side eu_flux_side(const eu_q &q, const eu_rcp &rr)
  * Bound by FP64 issue: about 200 instructions, four of them transcendental
  * (three square-root estimates and 1/(sl + sr); the reciprocals of the L, R
  * and Roe densities come from their roots), for 17 quotients.  Against
- * reciprocal instructions and two Newton steps for every denominator,
- * separate limiter differences per side and halvings as operations of their
- * own, a band-kernel cell and stage went from 605 to 482 VALU instructions:
- * Euler 1024^2 72.2 -> 57.2 us a step, 2048^2 FP32 state 223 -> 175, standard
- * kernel 1000 x 1500 108 -> 92.6, bitwise equal. */
+ * reciprocal instructions for every denominator, separate limiter differences per side and halvings as operations of their
+ * own, a band-kernel cell and stage went from 605 to 482 VALU instructions
+ * (488 with eu_recip's last step as it is now): Euler 1024^2 72.2 -> 57.2 us a
+ * step, 2048^2 FP32 state 223 -> 175, standard kernel 1000 x 1500 108 -> 92.6,
+ * bitwise equal. */
 template <bool XDIR>
 __device__ __forceinline__ void eu_face_vals(const eu_q &a, const eu_q &b, double cl, double cr, eu_q &f, eu_q &d)
 {
@@ -319,7 +336,7 @@ __device__ __forceinline__ void eu_face_vals(const eu_q &a, const eu_q &b, doubl
     (XDIR ? f.n : f.m) = l.c + r.c;
     f.e = l.e + r.e;
     const double sl = wl.s, sr = wr.s;
-    const double den = eu_quo_pos(1.0, eu_recip(sl + sr));
+    const double den = eu_inverse(sl + sr);
     const double a0 = sl * sr;
     const double a1 = (sl * eu_quo_pos(L.m, rl) + sr * eu_quo_pos(R.m, rr)) * den;
     const double a2 = (sl * eu_quo_pos(L.n, rl) + sr * eu_quo_pos(R.n, rr)) * den;
