@@ -956,7 +956,7 @@ class Engine:
         # same spec (kernels.load), so the owner of their constants is kept
         # on the modules themselves; any constant write clears it.
         if any(m.const_owner is not t for m in mods):
-            cls.cpu.set_globals(*t.problem.globals, source_mod=plugins.SourceModuleFacade(mods))
+            cls.cpu.set_globals(*t.problem.globals, source_mod=plugins.SourceModuleFacade(mods, wait=False))
             for m in mods:
                 m.const_owner = t
         G, P, T = t.times.G, cls.P, t.T

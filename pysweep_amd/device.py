@@ -14,12 +14,13 @@ import numpy
 from pysweep_amd import hip, kernels, plugins, schedule
 
 
-def range_fault(modules, clear=False):
+def range_fault(modules, clear=False, wait=True):
     """Whether a plugin that checks its division range (the Euler plugin's
     EU_RANGE_FAULT) met a state outside it in any of ``modules`` since the
-    last clear (waits for the work stream); ``clear`` resets the flags
-    instead, in stream order.  Modules without the flag never report one."""
-    hit = False
+    last clear; ``clear`` resets the flags instead.  Both wait for the work
+    stream; a clear with ``wait=False`` is only queued on it.  Modules without
+    the flag never report one."""
+    hit = queued = False
     for m in modules:
         try:
             ptr, _ = m.get_global("EU_RANGE_FAULT")
@@ -27,10 +28,13 @@ def range_fault(modules, clear=False):
             continue
         if clear:
             hip.memset_async(ptr, 0, 4)
+            queued = True
         else:
             v = numpy.zeros(1, numpy.int32)
             hip.dtoh(v, ptr)
             hit = hit or bool(v[0])
+    if queued and wait:
+        hip.synchronize()
     return hit
 
 
@@ -47,9 +51,12 @@ class _Run:
     def facade(self):
         return plugins.SourceModuleFacade(self.modules)
 
-    def set_globals(self, cpu_module, globals_):
-        """The plugin writes its device constants into every module."""
-        cpu_module.set_globals(*globals_, source_mod=self.facade())
+    def set_globals(self, cpu_module, globals_, wait=True):
+        """The plugin writes its device constants into every module (on the
+        device on return; with ``wait=False`` queued on the work stream)."""
+        cpu_module.set_globals(*globals_, source_mod=plugins.SourceModuleFacade(self.modules, wait=False))
+        if wait:
+            hip.synchronize()
 
     def poison(self):
         """Fill every level of the ring with NaN (all bytes 0xFF, a NaN in
@@ -63,9 +70,13 @@ class _Run:
         if ic.shape != (self.nv, self.nx, self.ny):
             raise ValueError(f"initial condition shape {ic.shape} != {(self.nv, self.nx, self.ny)}")
         first = self.ring.ptr
-        self.ring.upload(ic)
+        if self.its == 1:
+            self.ring.upload(ic)
+            return
+        hip.htod_async(first, ic)
         for A in range(1, self.its):  # one copy over the bus; the others stay on the device
             hip.dtod_async(first + (A % self.T) * self.level_bytes, first, self.level_bytes)
+        hip.synchronize()
 
     def keep_ic_on_device(self, ic):
         """Device copy of the initial condition for stream-ordered resets."""
@@ -88,10 +99,10 @@ class _Run:
         out[...] = buf
         return out
 
-    def range_fault(self, clear=False):
+    def range_fault(self, clear=False, wait=True):
         """Whether the plugin met a state outside its division range in any
         of the run's modules since the last clear (``range_fault``)."""
-        return range_fault(self.modules, clear)
+        return range_fault(self.modules, clear, wait)
 
     def sums(self, A):
         """FP64 (sums, sums of magnitudes) of level A's variables, summed on

@@ -437,6 +437,13 @@ def htod(dptr, arr):
     check(_htod(dptr, a.ctypes.data, a.nbytes), "ps_memcpy_htod")
 
 
+def htod_async(dptr, arr):
+    """Queue the copy of a contiguous numpy array to device memory; the array
+    stays as it is until the work stream has been waited for."""
+    assert arr.flags.c_contiguous
+    check(_htod_async(dptr, arr.ctypes.data, arr.nbytes), "ps_memcpy_htod_async")
+
+
 def dtoh(out, dptr):
     """Copy out.nbytes bytes from device address dptr into the contiguous
     numpy array ``out`` (waits for the work stream)."""

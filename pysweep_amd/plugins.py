@@ -21,11 +21,14 @@ import numpy
 class GlobalHandle:
     """A device global that may exist in several compiled modules (the swept
     and standard kernels are separate compilations of the same plugin
-    source); writes go to every copy."""
+    source); writes go to every copy.  ``wait``: a write has reached the
+    device when it returns, as PyCUDA's; without it writes are queued on the
+    calling thread's current context, whose owner waits."""
 
-    def __init__(self, name, copies):
+    def __init__(self, name, copies, wait=True):
         self.name = name
         self.copies = copies  # list of (device pointer, size in bytes)
+        self.wait = wait
 
     @property
     def nbytes(self):
@@ -79,6 +82,8 @@ class _Driver:
                 if len(data) > n:
                     raise ValueError(f"{len(data)} bytes do not fit device global {dst.name!r} ({n} bytes)")
                 _hip().write_bytes(ptr, data)
+            if dst.wait:
+                _hip().synchronize()
         else:
             _hip().htod_bytes(int(dst), data)
 
@@ -102,10 +107,12 @@ driver = _Driver()
 
 class SourceModuleFacade:
     """What a plugin's ``set_globals(..., source_mod=...)`` receives: the
-    compiled device modules of one plugin source."""
+    compiled device modules of one plugin source (``wait``: see
+    ``GlobalHandle``)."""
 
-    def __init__(self, modules):
+    def __init__(self, modules, wait=True):
         self.modules = list(modules)
+        self.wait = wait
 
     def get_global(self, name):
         copies = [m.get_global(name) for m in self.modules]
@@ -113,7 +120,7 @@ class SourceModuleFacade:
             # a plugin writes its constants through this handle: whoever
             # recorded the module's constants as theirs no longer owns them
             m.const_owner = None
-        h = GlobalHandle(name, copies)
+        h = GlobalHandle(name, copies, self.wait)
         return h, h.nbytes
 
     def get_function(self, name):

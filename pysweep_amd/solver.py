@@ -298,11 +298,12 @@ class Solver(object):
                                            generic=t.get("generic", False), defines=defines)
         # CPU globals, then the plugin's device constants (core/block.py:50, 90)
         self.cpu.set_globals(*self.globals)
-        self._run.set_globals(self.cpu, self.globals)
+        # (both queued: the upload behind them waits for the work stream)
+        self._run.set_globals(self.cpu, self.globals, wait=False)
+        self._run.range_fault(clear=True, wait=False)
         if t.get("poison"):
             self._run.poison()
         self._run.upload_ic(self.initialConditions)
-        self._run.range_fault(clear=True)
         # FP64 sums of the conserved quantities at the start (device-side;
         # read with the final level's)
         self._run.sums_async(self.intermediate - 1, 0)
