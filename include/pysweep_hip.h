@@ -35,7 +35,10 @@ typedef void *ps_event;    /* timing event (hipEvent_t)           */
 typedef void *ps_graph;    /* instantiated graph (hipGraphExec_t) */
 typedef void *ps_context;  /* device + work stream + launch timer */
 
-/* ABI version of this header. */
+/* ABI version of this header: changes with the plans' layout, the entry
+ * points or the kernels' arguments; a caller compiled against another one has
+ * to be rebuilt. */
+#define PS_VERSION 7
 int ps_version(void);
 
 /* Message of the last failure on this thread ("" if none). */

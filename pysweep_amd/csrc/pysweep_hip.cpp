@@ -336,7 +336,7 @@ int level_sums(const void *level, int fp32, int nv, size_t cells, double *sums, 
 
 extern "C" {
 
-int ps_version(void) { return 6; }
+int ps_version(void) { return PS_VERSION; }
 
 const char *ps_last_error(void) { return g_error.c_str(); }
 

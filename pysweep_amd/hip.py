@@ -25,6 +25,20 @@ if not os.path.exists(LIBPATH):
 
 _lib = ctypes.CDLL(LIBPATH)
 
+#: PS_VERSION of the header that the structures below follow
+ABI_VERSION = 7
+
+
+def check_abi(version):
+    """Refuse a library built from another version of the header: its plans
+    and kernel arguments are laid out differently."""
+    if version != ABI_VERSION:
+        raise ImportError(f"{LIBPATH} has interface version {version}, this package needs {ABI_VERSION}: "
+                          "build it again with __graft_entry__.build() or python -m pysweep_amd.build")
+
+
+check_abi(_lib.ps_version())
+
 c_int, c_size_t, c_void_p, c_char_p = ctypes.c_int, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_char_p
 
 
