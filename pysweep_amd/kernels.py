@@ -311,8 +311,9 @@ def has_band_chain(user_path):
 
 def band_has_full(spec):
     """Whether a band module has a kernel of its own for whole launches
-    (BandFull: the point-update plugins)."""
-    return spec.kind == "band" and not spec.multi and has_point_update(spec.user_path)
+    (BandFull: the point-update plugins without a sweep of their own)."""
+    return (spec.kind == "band" and not spec.multi and has_point_update(spec.user_path) and
+            not has_band_sweep(spec.user_path))
 
 
 def band_full_rows(spec, nx, ny, simds=BAND_SIMDS):
