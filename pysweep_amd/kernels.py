@@ -360,11 +360,13 @@ def band_launch(spec, nx, ny, rows=None):
     if spec.multi or not has_band_chain(spec.user_path):
         rows = int(rows or band_rows(spec, nx, ny))
         return rows, {"rows": rows, "chain": 0}
-    if rows is None:
-        rows, chain = band_chain_rows(spec, nx, ny)
-    else:
+    if rows is not None:
         rows = int(rows)
-        rows, chain = (BAND_CHAIN * rows - 2, BAND_CHAIN) if rows >= 7 else (rows, 0)
+        if rows < 7:
+            return rows, {"rows": rows, "chain": 0}
+        # (no longer than the grid: four segments may be beyond 32 bits)
+        return rows, {"rows": min(BAND_CHAIN * rows - 2, nx), "chain": BAND_CHAIN}
+    rows, chain = band_chain_rows(spec, nx, ny)
     return -(-(rows + 2) // BAND_CHAIN) if chain else rows, {"rows": rows, "chain": chain}
 
 
