@@ -251,7 +251,8 @@ class BandRun(_Run):
     equal."""
 
     def __init__(self, cu_path, nv, ops, its, nx, ny, levels=None, rows=None, real="double", defines=()):
-        self.spec = kernels.band_spec(cu_path, nv, ops, its, real=real, levels=levels, defines=defines)
+        self.spec = kernels.band_spec(cu_path, nv, ops, its, real=real, levels=levels,
+                                      defines=kernels.band_defines(cu_path, ny, real, defines))
         super().__init__(nv, its, nx, ny, self.spec.levels + its, real)
         mod = kernels.load(self.spec)
         self.modules = [mod]

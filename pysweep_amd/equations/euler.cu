@@ -825,6 +825,13 @@ __device__ __forceinline__ void eu_band_xface(const eu_band_win<R> &w, eu_q &xc)
 
 #define EU_GLOBAL __attribute__((address_space(1)))
 
+/* byte offset of a column */
+#ifdef PS_BAND_WIDE
+typedef size_t eu_band_off;
+#else
+typedef unsigned eu_band_off;
+#endif
+
 template <class R>
 struct eu_band_ctx {
     /* the ring in the global address space: its accesses compile to global
@@ -835,7 +842,7 @@ struct eu_band_ctx {
     size_t cells;
     int s0, T, nx, ny, wlo, hh;
     int n, e1;         /* rows of the segment; level 1 is computed until step e1 */
-    unsigned col, oc;  /* this lane's column in bytes; the same unwrapped */
+    eu_band_off col, oc;  /* this lane's column in bytes; the same unwrapped */
     bool out_col;
 };
 
@@ -844,15 +851,15 @@ struct eu_band_ctx {
  * empty asm statements keep it so: the compiler would carry the column as a
  * 64-bit number around the loop and add every row to it in vector
  * instructions, 6 a cell. */
-__device__ __forceinline__ unsigned eu_band_lane(unsigned bytes)
+__device__ __forceinline__ eu_band_off eu_band_lane(eu_band_off bytes)
 {
-    unsigned o;
+    eu_band_off o;
     asm volatile("" : "=v"(o) : "0"(bytes));
     return o;
 }
 
 template <class T>
-__device__ __forceinline__ T *eu_band_at(T *row, unsigned bytes)
+__device__ __forceinline__ T *eu_band_at(T *row, eu_band_off bytes)
 {
     typedef EU_GLOBAL char B;
     asm("" : "+s"(row));
@@ -862,7 +869,7 @@ __device__ __forceinline__ T *eu_band_at(T *row, unsigned bytes)
 template <class R>
 __device__ __forceinline__ void eu_band_load(const eu_band_ctx<R> &c, int row, eu_band_row<R> &o)
 {
-    const unsigned col = eu_band_lane(c.col);
+    const eu_band_off col = eu_band_lane(c.col);
 #pragma unroll
     for (int v = 0; v < 4; ++v) o.v[v] = *eu_band_at(c.in + (v * c.cells + (size_t)row * c.ny), col);
 }
@@ -872,7 +879,7 @@ __device__ __forceinline__ void eu_band_store(const eu_band_ctx<R> &c, int l, in
 {
     const int slot = c.s0 + l >= c.T ? c.s0 + l - c.T : c.s0 + l;
     if (c.out_col) {
-        const unsigned col = eu_band_lane(c.oc);
+        const eu_band_off col = eu_band_lane(c.oc);
 #pragma unroll
         for (int v = 0; v < 4; ++v)
             *eu_band_at(c.state + (((size_t)slot * NV + v) * c.cells + (size_t)row * c.ny), col) = o.v[v];
@@ -975,8 +982,8 @@ __device__ __forceinline__ void eu_band_segment(R *state, int A, const ps_band_g
     c.e1 = n + (g.hh >= 2 && !nxt ? 8 : 4);
     const int o = lane - 2 * PS_BAND_H;  /* band-local output column */
     c.out_col = o >= 0 && o < WOUT && band * WOUT + o < g.ny;
-    c.oc = (unsigned)(band * WOUT + o) * (unsigned)sizeof(R);
-    c.col = (unsigned)eu_band_wrap(band * WOUT + o, g.ny) * (unsigned)sizeof(R);
+    c.oc = (eu_band_off)(band * WOUT + o) * (eu_band_off)sizeof(R);
+    c.col = (eu_band_off)eu_band_wrap(band * WOUT + o, g.ny) * (eu_band_off)sizeof(R);
     /* defined values in what the first steps read before any level has
      * produced it (never used by a valid cell) */
     eu_band_win<R> w0, w1;

@@ -470,6 +470,14 @@ def band_multi_rows(spec, shapes, simds=BAND_SIMDS):
     return [int(r) for r in best[1]]
 
 
+def band_defines(user_path, ny, real, defines=()):
+    """Macros of a one-problem band module for rows of ny columns: a plugin's
+    own sweep may keep its lanes' columns as 32-bit byte offsets unless
+    PS_BAND_WIDE says that a row is longer."""
+    wide = has_band_sweep(user_path) and ny * (8 if real == "double" else 4) > 1 << 32
+    return tuple(defines) + (("PS_BAND_WIDE",) if wide else ())
+
+
 def band_spec(user_path, nv, ops, its, real="double", levels=None, defines=(), multi=False):
     """The band module of a plugin; ``multi``: its instance-table form
     (BandMulti, one wavefront per workgroup)."""
