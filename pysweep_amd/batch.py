@@ -650,9 +650,11 @@ class _ClassTable:
         """Rounds between BandMulti launches: a host step's rounds are whole
         launches of every band-method problem (``Engine._band_rounds``), so
         all of a class begin theirs on the same rounds, and on the others (1
-        of 2 for Euler, 11 of 12 for heat) each work item would leave at once.
-        0, a launch on every round, where they do not or where a captured
-        graph is no whole number of launches."""
+        of 2 for Euler, 7 of 8 for heat with 32-bit state, 11 of 12 for heat)
+        each work item would leave at once.  0, a launch on every round, where
+        they do not or where a captured graph is no whole number of launches:
+        the default graphs of 8 rounds hold none of heat's 12 levels, whose
+        idle rounds therefore stay."""
         h = self.cls.band_h
         if not banded or any((t.c - 1) % h for t in banded) or graph_rounds % h:
             return 0
@@ -723,7 +725,7 @@ class Engine:
 
     ``band_solo``: a problem running alone takes its standard stages on the
     band kernel where that outruns the standard kernel (heat at every size,
-    Euler from 1024^2 cells: ``kernels.band_beats_standard``), in whole RK2
+    Euler from 640^2 cells: ``kernels.band_beats_standard``), in whole RK2
     steps, the stages before the first full step on the standard kernel;
     results are bitwise unchanged.
 

@@ -292,7 +292,7 @@ def launch_info(run):
     """Registers / LDS of the loaded kernels (for reports)."""
     out = {}
     for m in run.modules:
-        for name in ("UpPyramid", "Octahedron", "Standard", "Band"):
+        for name in ("UpPyramid", "Octahedron", "Standard", "Band", "BandFull"):
             try:
                 out[name] = hip.function_info(m.get_function(name))
             except Exception:

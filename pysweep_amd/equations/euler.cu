@@ -109,8 +109,9 @@ __device__ __forceinline__ eu_q eu_at(const S &s, int i)
  * up; a uniform stream's densities are such numbers.  eu_recip_from sees to it
  * whatever the estimates.  Of what is cheaper, one third-order step from the
  * hardware's estimate, y + y*(e + e*e), left some quotients one ulp off for k
- * around 2^27 sqrt(m), two Newton steps for k = 5 (the numerators hardest to
- * round, found on MI355X).  Against the third-order step the two instructions
+ * around 2^27 sqrt(m), two Newton steps, as the compiler's n / d takes them,
+ * for k = 5, 11 and 13 (the numerators hardest to round, found on MI355X, where
+ * n / d itself misses those three).  Against the third-order step the two instructions
  * more cost 1.8 % (Euler 1024^2 53.1 -> 54.1 us a step, standard kernel
  * 1000 x 1500 83.6 -> 85.1).
  */

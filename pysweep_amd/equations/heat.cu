@@ -19,8 +19,8 @@ __device__ __constant__ double ALPHA;
 __device__ __constant__ double COURANT;
 __device__ __constant__ int SCHEME; /* 1: forward Euler, 0: RK2 */
 
-/* COURANT*(p - 2c + m).  2c is exact, so p - 2c is one fused operation with
- * the same rounding. */
+/* COURANT*(p - 2c + m).  2c is exact (below 2^1023), so p - 2c is one fused
+ * operation with the same rounding. */
 __device__ __forceinline__ double heat_second(double p, double c, double m)
 {
     return COURANT * (__builtin_fma(-2.0, c, p) + m);

@@ -213,13 +213,17 @@ def band_multi_levels(user_path, its, real="double"):
 #: 2-column halo per level) is taken to be the faster swept kernel: its
 #: 64-column bands leave small grids too few wavefronts.
 BAND_SWEEP_MIN_CELLS = 1 << 17
-#: A sweep in chains (Euler's) is faster than the phase kernels on smaller
-#: grids too, measured on MI355X (Euler, 60 steps, us, band / phase kernels
-#: b=16): 16^2 687 / 1004, 128^2 734 / 1052, 192^2 772 / 1093, 240x272 901 /
-#: 1128, 256^2 917 / 1102, 288^2 972 / 1360, 352^2 1115 / 1404; 16x4064 891 /
-#: 1114, but 4064x16 1153 / 1100: there most of a band's columns are padding,
-#: so the cells with it count.  It takes the grids outside BAND_CHAIN_GAP:
-#: there it gains least, and 256^2 is tested to run on the phase kernels.
+#: A sheared sweep (one with chains, Euler's; on small grids its wavefronts
+#: work by themselves, one to six rows each) is faster than the phase kernels
+#: on smaller grids too, measured on MI355X (Euler, us a step, band / phase
+#: kernels b=16): 16^2 11.7 / 16.9, 128^2 12.4 / 17.7, 192^2 13.1 / 18.4,
+#: 240x272 15.5 / 19.4, 256^2 15.6 / 18.7, 256x272 15.7 / 22.7, 288^2 16.4 /
+#: 23.0, 352^2 18.7 / 23.9; 16x4064 15.4 / 19.1, but 4064x16 19.7 / 18.7: there
+#: most of a band's columns are padding, so the cells with it count.  With a
+#: history, every step handed to a callback (a launch per step either way):
+#: 16^2 11.8 / 17.1, 128^2 12.3 / 18.0, 240x272 15.5 / 19.6, 352^2 18.5 / 24.3,
+#: 4064x16 19.6 / 19.0.  BAND_CHAIN_GAP is no crossover (256^2 lies in it): it
+#: keeps the sizes around 256^2, whose kernel tests fix, on the phase kernels.
 BAND_CHAIN_GAP = (1 << 16, 5 << 14)
 #: cells from which the Euler band sweep outruns the standard kernel (us a
 #: step, band / standard with its 15-row tiles: 384^2 18.2 / 15.5, 512^2 24.5
@@ -269,16 +273,20 @@ BAND_SIMDS = 1024
 
 
 def band_rows(spec, nx, ny, simds=BAND_SIMDS):
-    """Output rows per wavefront for a band launch over nx x ny: the row
-    segment minimising the busiest SIMD's time (the larger segment on a
-    tie).  That SIMD runs m = ceil(wavefronts / SIMDs) wavefronts.  A
+    """Output rows per wavefront for a band launch over nx x ny of
+    wavefronts by themselves with a halo at both ends of a segment: the
+    point update's partial launches and histories, and plugin sweeps without
+    chains (whole launches: ``band_full_rows``; Euler: ``band_chain_rows``).
+    The row segment minimises the busiest SIMD's time (the larger segment on
+    a tie).  That SIMD runs m = ceil(wavefronts / SIMDs) wavefronts.  A
     wavefront's steps are its segment plus the x halo of the launch, rounded
     up to the step loop's unrolling (3); level l computes from the step its
     first valid row appears on; a few steps' worth of set-up is added.  Two
     or more wavefronts share their SIMD's issue slots in full; one alone
     stalls on its own dependences and issues about 0.815 of the time.  The
     constants are fitted to these MI355X measurements, whose ranking the
-    model reproduces (GCUPS): Euler 1024^2, rows 12 11.2, 16 10.0, 18 8.8,
+    model reproduces (GCUPS; the Euler sweep's before it was sheared): Euler
+    1024^2, rows 12 11.2, 16 10.0, 18 8.8,
     20 12.0, 22 12.3, 24 11.1, 28 10.2; Euler 2048^2, rows 16 15.9, 20 15.6,
     24 14.2, 26 16.0, 28 16.3, 32 14.2; heat 8192^2 at 12 levels, rows 64
     1833, 128 1970, 192 1868, 256 1856."""
@@ -382,11 +390,11 @@ def band_chain_rows(spec, nx, ny, simds=BAND_SIMDS):
     each m; a launch adds about 4.5 units, a chain's barrier and one-level
     steps another 0.8, and chains that fill the chip to the last workgroup
     share CUs (640^2: 252 chains 31.2 us, 240 27.7).  Measured (us a step,
-    chosen / best of the other form): 384^2 3 rows each 18.2 / 24.1, 512^2 6
-    rows 24.2 / 24.9, 640^2 chains of 32 27.7 / 29.1, 1024^2 chains of 41
-    53.0 / 55.6, 1424 x 1128 65 76.5 / 83.6, 2048^2 158 177.1 / 176.8, 4096^2
-    152 rows each 691 / 691.  Against segments that recompute both ends
-    (band_rows): 1024^2 56.7, 2048^2 181.3."""
+    chosen / best of the other form): 384^2 3 rows each 17.4 / 29.8, 512^2 6
+    rows 24.1 / 27.7, 640^2 chains of 32 27.9 / 29.3, 1024^2 chains of 40
+    54.8 / 55.8, 1424 x 1128 62 76.8 / 81.6, 2048^2 158 180.3 / 183.9, 4096^2
+    152 rows each 706 / 706.  Segments that recompute both ends (band_rows)
+    took 56.7 at 1024^2 where chains took 53.0."""
     bands = -(-ny // band_out_columns(spec))
     best = (float("inf"), min(nx, 128), 0)
     for m in range(1, 33):
